@@ -22,6 +22,7 @@
 #include <mutex>
 
 #include "../../include/trianglemix.h"
+#include "trianglemix_internal.h"
 #include "trianglemix_kernel.h"
 
 static_assert(TM_WORKSPACE_COUNTER_BYTES == tmx::kCounterBytes, "the public counter block size is the kernel's");
@@ -540,6 +541,70 @@ int launch(bool sparse, const void* query, const void* key_cache, const void* va
   return TM_OK;
 }
 
+int launched(hipError_t err) {
+  if (err == hipSuccess) return TM_OK;
+  return fail(TM_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+}
+
+// Checks of a paged KV write; index is the slot mapping or block table
+// (index_bytes long) the slots come from.  TM_OK with num_tokens == 0 means
+// nothing to write, whatever the pointers.
+int check_kv_write(const void* key, const void* value, const void* key_cache, const void* value_cache,
+                   const void* index, int64_t index_bytes, int64_t num_tokens, int64_t key_stride,
+                   int64_t value_stride, int64_t num_pages) {
+  g_last_error[0] = '\0';
+  if (num_tokens < 0 || num_tokens > tmx::kMaxPositions) {
+    return fail(TM_ERR_INVALID_ARGUMENT, "key and value must be [num_tokens, 8, 128] with 0 <= num_tokens <= %lld",
+                (long long)tmx::kMaxPositions);
+  }
+  if (num_pages <= 0) {
+    return fail(TM_ERR_INVALID_ARGUMENT, "key_cache must be [pages, 128, 8, 128] with pages > 0");
+  }
+  if (num_pages > tmx::kMaxPages) {
+    return fail(TM_ERR_UNSUPPORTED, "key_cache has %lld pages; the limit is %lld", (long long)num_pages,
+                (long long)tmx::kMaxPages);
+  }
+  if (num_tokens == 0) return TM_OK;
+  if (!key || !value || !key_cache || !value_cache || !index) {
+    return fail(TM_ERR_INVALID_ARGUMENT, "key, value, key_cache, value_cache and slot_mapping must be non-null");
+  }
+  constexpr int64_t kRowElems = int64_t(tmx::kKvHeads) * tmx::kHeadDim;
+  if (key_stride < kRowElems || value_stride < kRowElems || key_stride % 8 != 0 || value_stride % 8 != 0) {
+    return fail(TM_ERR_INVALID_ARGUMENT,
+                "key and value rows must hold [8, 128] contiguous elements with a row stride >= 1024 that is a "
+                "multiple of 8");
+  }
+  const uintptr_t misaligned = ((uintptr_t)key | (uintptr_t)value | (uintptr_t)key_cache | (uintptr_t)value_cache) & 15;
+  if (misaligned) {
+    return fail(TM_ERR_INVALID_ARGUMENT, "key, value and the caches must be 16-byte aligned");
+  }
+  // The caches are written: they must not overlap each other, the sources or the slot source.
+  const Range r_k{(uintptr_t)key, (uintptr_t)key + uintptr_t(((num_tokens - 1) * key_stride + kRowElems) * 2)};
+  const Range r_v{(uintptr_t)value, (uintptr_t)value + uintptr_t(((num_tokens - 1) * value_stride + kRowElems) * 2)};
+  const Range r_kc{(uintptr_t)key_cache, (uintptr_t)key_cache + uintptr_t(num_pages * kPageBytes)};
+  const Range r_vc{(uintptr_t)value_cache, (uintptr_t)value_cache + uintptr_t(num_pages * kPageBytes)};
+  const Range r_s{(uintptr_t)index, (uintptr_t)index + uintptr_t(index_bytes)};
+  if (overlaps(r_kc, r_vc) || overlaps(r_kc, r_k) || overlaps(r_kc, r_v) || overlaps(r_kc, r_s) ||
+      overlaps(r_vc, r_k) || overlaps(r_vc, r_v) || overlaps(r_vc, r_s)) {
+    return fail(TM_ERR_INVALID_ARGUMENT,
+                "key_cache and value_cache must not overlap each other, key, value or slot_mapping");
+  }
+  return TM_OK;
+}
+
+// The block table covers logical tokens first_token .. + num_tokens - 1 (the kernels read it unchecked).
+int check_chunk_table(int64_t table_cols, int64_t first_token, int64_t num_tokens) {
+  if (first_token < 0 || num_tokens < 0 || first_token > tmx::kMaxPositions - num_tokens ||
+      num_tokens > tmx::kMaxPositions) {
+    return fail(TM_ERR_INVALID_ARGUMENT, "first_token and num_tokens must be non-negative and at most %lld in sum",
+                (long long)tmx::kMaxPositions);
+  }
+  if (num_tokens > 0 && (first_token + num_tokens - 1) / tmx::kPageSize >= table_cols) {
+    return fail(TM_ERR_INVALID_ARGUMENT, "block_table lacks logical pages required by the chunk");
+  }
+  return TM_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -651,50 +716,32 @@ void tm_plan_override(int32_t kv_parts, int32_t tiles_per_split) {
 int tm_reshape_and_cache(const void* key, const void* value, void* key_cache, void* value_cache,
                          const int64_t* slot_mapping, int64_t num_tokens, int64_t key_stride, int64_t value_stride,
                          int64_t num_pages, void* stream) {
+  const int st = check_kv_write(key, value, key_cache, value_cache, slot_mapping, num_tokens * 8, num_tokens,
+                                key_stride, value_stride, num_pages);
+  if (st != TM_OK || num_tokens == 0) return st;  // 0 tokens: nothing to write, nothing enqueued
+  return launched(tmx::launch_paged_kv_write(key, value, key_cache, value_cache, slot_mapping, num_tokens, key_stride,
+                                             value_stride, num_pages, static_cast<hipStream_t>(stream)));
+}
+
+int tmi_write_chunk_kv(const void* key, const void* value, void* key_cache, void* value_cache,
+                       const int32_t* block_table, int64_t table_cols, int64_t first_token, int64_t num_tokens,
+                       int64_t key_stride, int64_t value_stride, int64_t num_pages, void* stream) {
+  int st = check_kv_write(key, value, key_cache, value_cache, block_table, table_cols * 4, num_tokens, key_stride,
+                          value_stride, num_pages);
+  if (st == TM_OK) st = check_chunk_table(table_cols, first_token, num_tokens);
+  if (st != TM_OK || num_tokens == 0) return st;
+  return launched(tmx::launch_chunk_kv_write(key, value, key_cache, value_cache, block_table, first_token, num_tokens,
+                                             key_stride, value_stride, num_pages, static_cast<hipStream_t>(stream)));
+}
+
+int tmi_chunk_slots(const int32_t* block_table, int64_t table_cols, int64_t first_token, int64_t num_tokens,
+                    int64_t* slots, void* stream) {
   g_last_error[0] = '\0';
-  if (num_tokens < 0 || num_tokens > tmx::kMaxPositions) {
-    return fail(TM_ERR_INVALID_ARGUMENT, "key and value must be [num_tokens, 8, 128] with 0 <= num_tokens <= %lld",
-                (long long)tmx::kMaxPositions);
-  }
-  if (num_pages <= 0) {
-    return fail(TM_ERR_INVALID_ARGUMENT, "key_cache must be [pages, 128, 8, 128] with pages > 0");
-  }
-  if (num_pages > tmx::kMaxPages) {
-    return fail(TM_ERR_UNSUPPORTED, "key_cache has %lld pages; the limit is %lld", (long long)num_pages,
-                (long long)tmx::kMaxPages);
-  }
-  if (num_tokens == 0) return TM_OK;  // nothing to write, nothing enqueued
-  if (!key || !value || !key_cache || !value_cache || !slot_mapping) {
-    return fail(TM_ERR_INVALID_ARGUMENT, "key, value, key_cache, value_cache and slot_mapping must be non-null");
-  }
-  constexpr int64_t kRowElems = int64_t(tmx::kKvHeads) * tmx::kHeadDim;
-  if (key_stride < kRowElems || value_stride < kRowElems || key_stride % 8 != 0 || value_stride % 8 != 0) {
-    return fail(TM_ERR_INVALID_ARGUMENT,
-                "key and value rows must hold [8, 128] contiguous elements with a row stride >= 1024 that is a "
-                "multiple of 8");
-  }
-  const uintptr_t misaligned = ((uintptr_t)key | (uintptr_t)value | (uintptr_t)key_cache | (uintptr_t)value_cache) & 15;
-  if (misaligned) {
-    return fail(TM_ERR_INVALID_ARGUMENT, "key, value and the caches must be 16-byte aligned");
-  }
-  // The caches are written: they must not overlap each other, the sources or the slot mapping.
-  const Range r_k{(uintptr_t)key, (uintptr_t)key + uintptr_t(((num_tokens - 1) * key_stride + kRowElems) * 2)};
-  const Range r_v{(uintptr_t)value, (uintptr_t)value + uintptr_t(((num_tokens - 1) * value_stride + kRowElems) * 2)};
-  const Range r_kc{(uintptr_t)key_cache, (uintptr_t)key_cache + uintptr_t(num_pages * kPageBytes)};
-  const Range r_vc{(uintptr_t)value_cache, (uintptr_t)value_cache + uintptr_t(num_pages * kPageBytes)};
-  const Range r_s{(uintptr_t)slot_mapping, (uintptr_t)slot_mapping + uintptr_t(num_tokens * 8)};
-  if (overlaps(r_kc, r_vc) || overlaps(r_kc, r_k) || overlaps(r_kc, r_v) || overlaps(r_kc, r_s) ||
-      overlaps(r_vc, r_k) || overlaps(r_vc, r_v) || overlaps(r_vc, r_s)) {
-    return fail(TM_ERR_INVALID_ARGUMENT,
-                "key_cache and value_cache must not overlap each other, key, value or slot_mapping");
-  }
-  const hipError_t err = tmx::launch_paged_kv_write(key, value, key_cache, value_cache, slot_mapping, num_tokens,
-                                                    key_stride, value_stride, num_pages,
-                                                    static_cast<hipStream_t>(stream));
-  if (err != hipSuccess) {
-    return fail(TM_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
-  }
-  return TM_OK;
+  const int st = check_chunk_table(table_cols, first_token, num_tokens);
+  if (st != TM_OK || num_tokens == 0) return st;
+  if (!block_table || !slots) return fail(TM_ERR_INVALID_ARGUMENT, "block_table and slots must be non-null");
+  return launched(
+      tmx::launch_chunk_slots(block_table, first_token, num_tokens, slots, static_cast<hipStream_t>(stream)));
 }
 
 }  // extern "C"

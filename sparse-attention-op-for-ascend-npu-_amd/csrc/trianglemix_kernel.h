@@ -146,6 +146,17 @@ hipError_t launch_paged_kv_write(const void* key, const void* value, void* key_c
                                  const int64_t* slot_mapping, int64_t num_tokens, int64_t key_stride,
                                  int64_t value_stride, int64_t num_pages, hipStream_t stream);
 
+// The same write for logical tokens first_token .. first_token + num_tokens -
+// 1 of the request with this block table: token t goes to slot block_table[t /
+// 128] * 128 + t % 128.
+hipError_t launch_chunk_kv_write(const void* key, const void* value, void* key_cache, void* value_cache,
+                                 const int32_t* block_table, int64_t first_token, int64_t num_tokens,
+                                 int64_t key_stride, int64_t value_stride, int64_t num_pages, hipStream_t stream);
+
+// Enqueues slots[i] = the slot above of token first_token + i.
+hipError_t launch_chunk_slots(const int32_t* block_table, int64_t first_token, int64_t num_tokens, int64_t* slots,
+                              hipStream_t stream);
+
 }  // namespace tmx
 
 #endif  // TRIANGLEMIX_KERNEL_H

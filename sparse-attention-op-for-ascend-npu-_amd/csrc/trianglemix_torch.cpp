@@ -22,6 +22,11 @@
 //
 //   trianglemix::reshape_and_cache(key, value, key_cache!, value_cache!, slot_mapping) -> ()
 //
+// with its single-request forms, the slots taken from the block table:
+//
+//   trianglemix::write_chunk_kv(key, value, key_cache!, value_cache!, block_table, query_start) -> ()
+//   trianglemix::chunk_slots(block_table, query_start, num_tokens) -> Tensor
+//
 // Input and output checks restate check_inputs / check_output (:29-97) with
 // the same predicates and messages ("GPU" for "NPU").  Launches go on the
 // current HIP stream of the query's device under a device guard, with no
@@ -52,6 +57,7 @@
 #include <vector>
 
 #include "../../include/trianglemix.h"
+#include "trianglemix_internal.h"
 
 namespace trianglemix_rocm {
 namespace {
@@ -199,27 +205,24 @@ at::Tensor& dense_paged_causal_attention_out(const at::Tensor& query, const at::
   return output;
 }
 
-// Paged KV write: token i's K / V rows go to cache slot slot_mapping[i]
-// (negative = padding, skipped).  key / value may be row-strided views (a
-// slice of a fused QKV buffer); their [8, 128] part must be contiguous.
-void reshape_and_cache(const at::Tensor& key, const at::Tensor& value, at::Tensor& key_cache, at::Tensor& value_cache,
-                       const at::Tensor& slot_mapping) {
-  TORCH_CHECK(key.is_cuda() && value.is_cuda() && key_cache.is_cuda() && value_cache.is_cuda() &&
-                  slot_mapping.is_cuda(),
+// Checks of a paged KV write; `index` (the slot mapping or the block table)
+// lies on the same device.  key / value may be row-strided views (a slice of
+// a fused QKV buffer); their [8, 128] part must be contiguous.
+void check_kv_write(const at::Tensor& key, const at::Tensor& value, const at::Tensor& key_cache,
+                    const at::Tensor& value_cache, const at::Tensor& index) {
+  TORCH_CHECK(key.is_cuda() && value.is_cuda() && key_cache.is_cuda() && value_cache.is_cuda() && index.is_cuda(),
               "key, value, key_cache, value_cache and slot_mapping must be GPU tensors");
   TORCH_CHECK(key.device() == value.device() && key.device() == key_cache.device() &&
-                  key.device() == value_cache.device() && key.device() == slot_mapping.device(),
+                  key.device() == value_cache.device() && key.device() == index.device(),
               "all inputs must be on the same GPU device");
   TORCH_CHECK(key.scalar_type() == at::ScalarType::BFloat16 && value.scalar_type() == at::ScalarType::BFloat16 &&
                   key_cache.scalar_type() == at::ScalarType::BFloat16 &&
                   value_cache.scalar_type() == at::ScalarType::BFloat16,
               "key, value, key_cache and value_cache must be BF16");
-  TORCH_CHECK(slot_mapping.scalar_type() == at::ScalarType::Long && slot_mapping.dim() == 1 &&
-                  slot_mapping.is_contiguous(),
-              "slot_mapping must be a contiguous INT64 [num_tokens] tensor");
-  TORCH_CHECK(key.dim() == 3 && key.size(1) == 8 && key.size(2) == 128 && value.sizes() == key.sizes(),
-              "key and value must be [num_tokens, 8, 128]");
-  TORCH_CHECK(key.size(0) == slot_mapping.size(0), "slot_mapping must hold one slot per token");
+}
+
+void check_kv_shapes(const at::Tensor& key, const at::Tensor& value, const at::Tensor& key_cache,
+                     const at::Tensor& value_cache) {
   TORCH_CHECK(key.stride(2) == 1 && key.stride(1) == 128 && value.stride(2) == 1 && value.stride(1) == 128,
               "the [8, 128] part of each key / value row must be contiguous");
   TORCH_CHECK(key_cache.dim() == 4 && key_cache.size(1) == 128 && key_cache.size(2) == 8 &&
@@ -232,6 +235,20 @@ void reshape_and_cache(const at::Tensor& key, const at::Tensor& value, at::Tenso
   at::assert_no_overlap(key_cache, value);
   at::assert_no_overlap(value_cache, key);
   at::assert_no_overlap(value_cache, value);
+}
+
+// Paged KV write: token i's K / V rows go to cache slot slot_mapping[i]
+// (negative = padding, skipped).
+void reshape_and_cache(const at::Tensor& key, const at::Tensor& value, at::Tensor& key_cache, at::Tensor& value_cache,
+                       const at::Tensor& slot_mapping) {
+  check_kv_write(key, value, key_cache, value_cache, slot_mapping);
+  TORCH_CHECK(slot_mapping.scalar_type() == at::ScalarType::Long && slot_mapping.dim() == 1 &&
+                  slot_mapping.is_contiguous(),
+              "slot_mapping must be a contiguous INT64 [num_tokens] tensor");
+  TORCH_CHECK(key.dim() == 3 && key.size(1) == 8 && key.size(2) == 128 && value.sizes() == key.sizes(),
+              "key and value must be [num_tokens, 8, 128]");
+  TORCH_CHECK(key.size(0) == slot_mapping.size(0), "slot_mapping must hold one slot per token");
+  check_kv_shapes(key, value, key_cache, value_cache);
   const int64_t num_tokens = key.size(0);
   if (num_tokens == 0) return;
   c10::OptionalDeviceGuard guard(key.device());
@@ -243,7 +260,57 @@ void reshape_and_cache(const at::Tensor& key, const at::Tensor& value, at::Tenso
   check_status(status, "reshape_and_cache");
 }
 
+void check_table(const at::Tensor& block_table) {
+  TORCH_CHECK(block_table.scalar_type() == at::ScalarType::Int && block_table.dim() == 2 && block_table.size(0) == 1 &&
+                  block_table.is_contiguous(),
+              "block_table must be a contiguous INT32 [1, max_pages] tensor");
+}
+
+// Cache slots of logical tokens query_start .. query_start + num_tokens - 1 of
+// the request with this block table.
+at::Tensor chunk_slots(const at::Tensor& block_table, int64_t query_start, int64_t num_tokens) {
+  TORCH_CHECK(block_table.is_cuda(), "block_table must be a GPU tensor");
+  check_table(block_table);
+  TORCH_CHECK(num_tokens >= 0, "num_tokens must be non-negative");
+  c10::OptionalDeviceGuard guard(block_table.device());
+  at::Tensor slots = at::empty({num_tokens}, block_table.options().dtype(at::kLong));
+  void* stream = c10::hip::getCurrentHIPStream(block_table.device().index()).stream();
+  const int status = tmi_chunk_slots(block_table.data_ptr<int32_t>(), block_table.size(1), query_start, num_tokens,
+                                     slots.data_ptr<int64_t>(), stream);
+  check_status(status, "chunk_slots");
+  return slots;
+}
+
+// reshape_and_cache of those tokens in one launch, without a slot mapping.
+void write_chunk_kv(const at::Tensor& key, const at::Tensor& value, at::Tensor& key_cache, at::Tensor& value_cache,
+                    const at::Tensor& block_table, int64_t query_start) {
+  check_kv_write(key, value, key_cache, value_cache, block_table);
+  check_table(block_table);
+  TORCH_CHECK(key.dim() == 3 && key.size(1) == 8 && key.size(2) == 128 && value.sizes() == key.sizes(),
+              "key and value must be [num_tokens, 8, 128]");
+  // A table inside the caches would be overwritten while it is read: map first.
+  if (at::get_overlap_status(key_cache, block_table) != at::MemOverlapStatus::No ||
+      at::get_overlap_status(value_cache, block_table) != at::MemOverlapStatus::No) {
+    reshape_and_cache(key, value, key_cache, value_cache, chunk_slots(block_table, query_start, key.size(0)));
+    return;
+  }
+  check_kv_shapes(key, value, key_cache, value_cache);
+  const int64_t num_tokens = key.size(0);
+  if (num_tokens == 0) return;
+  c10::OptionalDeviceGuard guard(key.device());
+  void* stream = c10::hip::getCurrentHIPStream(key.device().index()).stream();
+  const int status = tmi_write_chunk_kv(key.data_ptr(), value.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
+                                        block_table.data_ptr<int32_t>(), block_table.size(1), query_start, num_tokens,
+                                        key.stride(0), value.stride(0), key_cache.size(0), stream);
+  check_status(status, "write_chunk_kv");
+}
+
 void meta_reshape_and_cache(const at::Tensor&, const at::Tensor&, at::Tensor&, at::Tensor&, const at::Tensor&) {}
+
+void meta_write_chunk_kv(const at::Tensor&, const at::Tensor&, at::Tensor&, at::Tensor&, const at::Tensor&, int64_t) {}
+at::Tensor meta_chunk_slots(const at::Tensor& block_table, int64_t, int64_t num_tokens) {
+  return at::empty({num_tokens}, block_table.options().dtype(at::kLong));
+}
 
 // Shape-only implementations (the reference's InferShape: out = query shape,
 // operator/op_host/triangle_paged_sparse_attention.cpp:332-346).
@@ -381,6 +448,10 @@ TORCH_LIBRARY_FRAGMENT(trianglemix, ops) {
   ops.def(
       "reshape_and_cache(Tensor key, Tensor value, Tensor(a!) key_cache, Tensor(b!) value_cache, "
       "Tensor slot_mapping) -> ()");
+  ops.def(
+      "write_chunk_kv(Tensor key, Tensor value, Tensor(a!) key_cache, Tensor(b!) value_cache, "
+      "Tensor block_table, int query_start) -> ()");
+  ops.def("chunk_slots(Tensor block_table, int query_start, int num_tokens) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(trianglemix, CUDA, ops) {
@@ -388,6 +459,8 @@ TORCH_LIBRARY_IMPL(trianglemix, CUDA, ops) {
   ops.impl("npu_triangle_paged_sparse_attention", &trianglemix_rocm::triangle_paged_sparse_attention_out);
   ops.impl("dense_paged_causal_attention.out", &trianglemix_rocm::dense_paged_causal_attention_out);
   ops.impl("reshape_and_cache", &trianglemix_rocm::reshape_and_cache);
+  ops.impl("write_chunk_kv", &trianglemix_rocm::write_chunk_kv);
+  ops.impl("chunk_slots", &trianglemix_rocm::chunk_slots);
 }
 
 TORCH_LIBRARY_IMPL(trianglemix, Meta, ops) {
@@ -395,4 +468,6 @@ TORCH_LIBRARY_IMPL(trianglemix, Meta, ops) {
   ops.impl("npu_triangle_paged_sparse_attention", &trianglemix_rocm::meta_out);
   ops.impl("dense_paged_causal_attention.out", &trianglemix_rocm::meta_dense_out);
   ops.impl("reshape_and_cache", &trianglemix_rocm::meta_reshape_and_cache);
+  ops.impl("write_chunk_kv", &trianglemix_rocm::meta_write_chunk_kv);
+  ops.impl("chunk_slots", &trianglemix_rocm::meta_chunk_slots);
 }

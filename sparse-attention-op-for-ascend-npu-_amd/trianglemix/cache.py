@@ -11,12 +11,23 @@ offset rule of the reference's harness, operator/tests/npu_v2_correctness.py:385
 from __future__ import annotations
 
 PAGE_SIZE = 128
+MAX_POSITIONS = 1 << 30  # the native ops' largest position
 
 
-def chunk_slot_mapping(block_table, query_start: int, num_tokens: int):
-    """int64 slots of logical tokens ``query_start .. query_start + num_tokens - 1`` (device of the table)."""
+def _native_table(block_table, query_start, *counts) -> bool:
+    """Whether the native ops take this block table as it is: a contiguous int32 GPU tensor and plain int
+    positions, with the adapter loaded.  Any other table (another dtype, a strided view, CPU, a tensor position)
+    goes through tensor operations."""
     import torch
 
+    from .native import triangle_mix_adapter_loaded
+
+    return (isinstance(block_table, torch.Tensor) and block_table.dtype is torch.int32 and block_table.is_cuda
+            and block_table.is_contiguous() and type(query_start) is int and all(type(n) is int for n in counts)
+            and query_start + sum(counts) <= MAX_POSITIONS and triangle_mix_adapter_loaded())
+
+
+def _check_chunk(block_table, query_start, num_tokens) -> None:
     if block_table.dim() != 2 or block_table.size(0) != 1:
         raise ValueError("block_table must be [1, max_pages]")
     if query_start < 0 or num_tokens < 0:
@@ -24,7 +35,16 @@ def chunk_slot_mapping(block_table, query_start: int, num_tokens: int):
     last = query_start + num_tokens
     if num_tokens and (last - 1) // PAGE_SIZE >= block_table.size(1):
         raise ValueError("block_table lacks logical pages required by the chunk")
-    t = torch.arange(query_start, last, dtype=torch.int64, device=block_table.device)
+
+
+def chunk_slot_mapping(block_table, query_start: int, num_tokens: int):
+    """int64 slots of logical tokens ``query_start .. query_start + num_tokens - 1`` (device of the table)."""
+    import torch
+
+    _check_chunk(block_table, query_start, num_tokens)
+    if _native_table(block_table, query_start, num_tokens):
+        return torch.ops.trianglemix.chunk_slots(block_table, query_start, num_tokens)
+    t = torch.arange(query_start, query_start + num_tokens, dtype=torch.int64, device=block_table.device)
     return block_table[0].to(torch.int64)[t // PAGE_SIZE] * PAGE_SIZE + t % PAGE_SIZE
 
 
@@ -40,5 +60,12 @@ def reshape_and_cache(key, value, key_cache, value_cache, slot_mapping) -> None:
 
 def write_chunk_kv(key, value, key_cache, value_cache, block_table, query_start: int) -> None:
     """Fill the pages of logical tokens ``query_start .. query_start + len(key) - 1``."""
-    reshape_and_cache(key, value, key_cache, value_cache,
-                      chunk_slot_mapping(block_table, query_start, key.shape[0]))
+    import torch
+
+    num_tokens = key.shape[0]
+    _check_chunk(block_table, query_start, num_tokens)
+    if _native_table(block_table, query_start, num_tokens):
+        # one launch: the kernel reads the slots from the block table
+        torch.ops.trianglemix.write_chunk_kv(key, value, key_cache, value_cache, block_table, query_start)
+        return
+    reshape_and_cache(key, value, key_cache, value_cache, chunk_slot_mapping(block_table, query_start, num_tokens))
