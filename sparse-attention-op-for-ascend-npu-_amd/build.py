@@ -86,7 +86,8 @@ def build_hip_library(phase_clocks: bool = False, plan_override: bool = False) -
     tmp = dst.with_suffix(".so.tmp")
     defines = (["-DTRIANGLEMIX_PHASE_CLOCKS"] if phase_clocks else []) + (["-DTRIANGLEMIX_PLAN_OVERRIDE"] if plan_override else [])
     _run([hipcc, *HIP_FLAGS, *defines, "-shared", f"-I{INCLUDE}",
-          str(CSRC / "trianglemix_kernel.hip"), str(CSRC / "trianglemix_cache.hip"), str(CSRC / "trianglemix_capi.cpp"),
+          str(CSRC / "trianglemix_kernel.hip"), str(CSRC / "trianglemix_wide.hip"), str(CSRC / "trianglemix_cache.hip"),
+          str(CSRC / "trianglemix_capi.cpp"),
           "-o", str(tmp)])
     _atomic_replace(tmp, dst)
     return dst

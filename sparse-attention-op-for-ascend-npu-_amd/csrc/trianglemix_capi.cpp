@@ -238,6 +238,7 @@ std::vector<int> split_candidates(int longest, int min_tiles, bool ladder_only) 
 
 struct ChunkPlan {
   int kv_parts, tiles_per_split;
+  bool wide;  // which kernel runs it (long_items below)
 };
 
 // The best (shape, T) among the shapes' candidates, in the order given
@@ -255,7 +256,7 @@ struct ShapeCandidates {
 ChunkPlan best_plan(const std::vector<int>& row_tiles, std::initializer_list<ShapeCandidates> shapes) {
   int longest = 0;
   for (const int n : row_tiles) longest = std::max(longest, n);
-  ChunkPlan best{0, 0};
+  ChunkPlan best{0, 0, false};
   double best_time = 0.0;
   for (const ShapeCandidates& s : shapes) {
     bool unsplit_done = false;  // every T >= longest is the same plan: simulate the first only
@@ -268,12 +269,12 @@ ChunkPlan best_plan(const std::vector<int>& row_tiles, std::initializer_list<Sha
       const double t = simulated_time(row_tiles, tk, *s.model,
                                       best.kv_parts == 0 ? std::numeric_limits<double>::infinity() : best_time);
       if (best.kv_parts == 0 || t < best_time) {
-        best = {s.kv_parts, tk};
+        best = {s.kv_parts, tk, false};
         best_time = t;
       }
     }
   }
-  if (best.kv_parts == 0) best = {shapes.begin()->kv_parts, std::max(longest, 1)};
+  if (best.kv_parts == 0) best = {shapes.begin()->kv_parts, std::max(longest, 1), false};
   return best;
 }
 
@@ -297,7 +298,7 @@ ChunkPlan choose_plan(const std::vector<int>& row_tiles, bool sparse) {
       if (tk < per_item || !layout_fits(split_layout(row_tiles, tk))) break;
       pick = tk;
     }
-    return {2, pick};
+    return {2, pick, false};
   }
   if (num_row_blocks >= kLargeMinRowBlocks) {
     return best_plan(row_tiles, {{2, &kLargeHalves, kLargeSplitTiles, false},
@@ -313,6 +314,46 @@ ChunkPlan choose_plan(const std::vector<int>& row_tiles, bool sparse) {
     return halves;
   }
   return best_plan(row_tiles, {{4, &kDenseQuarters, kMinSplitTiles, false}});
+}
+
+// Which kernel runs a plan: the one with 64 rows per wave
+// (trianglemix_wide.hip) when the plan's longest item has at least this many
+// loop iterations (tiles / KV parts), the eight-wave one otherwise.  The first
+// has the cheaper loop, the second the shorter start-up and merge, so the line
+// lies where the loop outweighs them, and higher where split rows merge in the
+// launch beside short sparse items.  Measured, us, eight-wave -> 64 rows per
+// wave, around each line:
+//  * KV quarters, nothing split or every row dense: 512 rows, longest item 4
+//    iterations 7.8 -> 7.9, 6 (split) 12.7 -> 12.7, 8 11.2 -> 10.7, 12 15.8 -> 14.7,
+//    32 39.0 -> 35.2;
+//  * KV quarters, split TriangleMix rows: 5 iterations 11.5 -> 13.0, 11 18.2 ->
+//    18.4 and 18.0 -> 19.1, 13 19.6 -> 21.1, 16 22.9 -> 19.8, 25.7 -> 23.7, 21
+//    29.8 -> 28.8;
+//  * KV halves: 9 iterations 13.6 -> 13.8, 14 (dense, split) 16.2 -> 15.8, 32
+//    40.0 -> 38.4, 64 104.5 -> 98.7; split TriangleMix rows: 11 16.9 -> 17.9,
+//    18 28.8 -> 29.7, 21 36.0 -> 35.0, 32 56.4 -> 55.5;
+//  * KV whole: 18 iterations 22.1 -> 21.6 and 20.2 -> 20.0, 576 557 -> 518;
+//    split, whose merge reads 66 KB per piece with two waves instead of four: 20
+//    iterations 43.1 -> 50.5, 64 101 -> 105, 144 147 -> 143, 256 308 -> 291.
+struct LongItems {
+  int unsplit, split;  // fewest iterations: nothing split or every row dense; split TriangleMix rows
+};
+constexpr LongItems kLongQuarters{8, 16};
+constexpr LongItems kLongHalves{14, 20};
+constexpr LongItems kLongWhole{16, 128};
+
+bool long_items(const std::vector<int>& row_tiles, const ChunkPlan& plan, bool sparse) {
+  int64_t longest = 0;  // tiles of the longest item
+  bool split = false, short_rows = false;
+  for (const int n : row_tiles) {
+    const int64_t pieces = (n + plan.tiles_per_split - 1) / plan.tiles_per_split;
+    longest = std::max(longest, (n + pieces - 1) / pieces);
+    split = split || pieces > 1;
+    short_rows = short_rows || pieces == 1;
+  }
+  const LongItems& least = plan.kv_parts == 4 ? kLongQuarters : (plan.kv_parts == 2 ? kLongHalves : kLongWhole);
+  const bool merges = split && (plan.kv_parts == 1 || (sparse && short_rows));
+  return (longest + plan.kv_parts - 1) / plan.kv_parts >= (merges ? least.split : least.unsplit);
 }
 
 // The choice depends only on the chunk geometry, which repeats for every layer
@@ -337,14 +378,15 @@ int g_override_parts = 0, g_override_tiles = 0;
 #endif
 
 ChunkPlan cached_plan(const PlanKey& key) {
-#ifdef TRIANGLEMIX_PLAN_OVERRIDE
-  if (g_override_parts > 0) return ChunkPlan{g_override_parts, g_override_tiles};
-#endif
   constexpr int kEntries = 64;
   thread_local PlanKey keys[kEntries];
   thread_local ChunkPlan values[kEntries];
   thread_local int used = 0, next = 0;
-  for (int i = 0; i < used; ++i) {
+  bool forced = false;
+#ifdef TRIANGLEMIX_PLAN_OVERRIDE
+  forced = g_override_parts > 0;
+#endif
+  for (int i = 0; i < used && !forced; ++i) {
     if (keys[i] == key) return values[i];
   }
   std::vector<int> row_tiles((size_t)key.num_row_blocks);
@@ -352,7 +394,16 @@ ChunkPlan cached_plan(const PlanKey& key) {
     row_tiles[(size_t)o] = tmx::row_block_splits((int)o, (int)key.num_row_blocks, (int)key.query_start,
                                                  (int)key.seq_len, (int)key.sparse_begin, (int)key.sparse_end, 1);
   }
-  const ChunkPlan plan = choose_plan(row_tiles, key.sparse_begin != 0);  // 0 only for the dense companion
+  const bool sparse = key.sparse_begin != 0;  // 0 only for the dense companion
+#ifdef TRIANGLEMIX_PLAN_OVERRIDE
+  if (forced) {
+    ChunkPlan plan{g_override_parts, g_override_tiles, false};
+    plan.wide = long_items(row_tiles, plan, sparse);
+    return plan;
+  }
+#endif
+  ChunkPlan plan = choose_plan(row_tiles, sparse);
+  plan.wide = long_items(row_tiles, plan, sparse);
   keys[next] = key;
   values[next] = plan;
   next = (next + 1) % kEntries;
@@ -366,6 +417,7 @@ constexpr int64_t kMaxItemsPerHead = int64_t(1) << 26;
 
 struct Geometry {
   int sparse_begin, sparse_end, num_row_blocks, tiles_per_split, kv_parts;
+  bool wide;
   int64_t items_per_head;
   int split_row_blocks;  // row blocks in issue order up to the last split one (0: nothing splits)
   int64_t split_items;   // their items: the partial records per KV head
@@ -379,6 +431,7 @@ Geometry make_geometry(bool sparse, int64_t query_tokens, int64_t query_start, i
   g.num_row_blocks = (int)((query_tokens + tmx::kRowBlock - 1) / tmx::kRowBlock);
   const ChunkPlan plan = cached_plan(PlanKey{g.num_row_blocks, query_start, seq_len, g.sparse_begin, g.sparse_end});
   g.kv_parts = plan.kv_parts;
+  g.wide = plan.wide;
   g.tiles_per_split = plan.tiles_per_split;
   int64_t items = 0;
   for (int o = 0; o < g.num_row_blocks; ++o) {
@@ -533,8 +586,8 @@ int launch(bool sparse, const void* query, const void* key_cache, const void* va
   p.split_row_blocks = g.split_row_blocks;
   p.split_items = (int)g.split_items;
   p.scale_log2 = scale * 1.4426950408889634f;
-  const hipError_t err =
-      tmx::launch_triangle_paged_attention(p, sparse, g.kv_parts, static_cast<hipStream_t>(stream));
+  const auto launch_kernel = g.wide ? tmx::launch_wide_attention : tmx::launch_triangle_paged_attention;
+  const hipError_t err = launch_kernel(p, sparse, g.kv_parts, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) {
     return fail(TM_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
   }
@@ -700,6 +753,13 @@ int tm_chunk_plan(int dense, int64_t query_tokens, int64_t query_start, int64_t 
   *tiles_per_split = g.tiles_per_split;
   *items_per_kv_head = g.items_per_head;
   return TM_OK;
+}
+
+int tmi_chunk_is_wide(int dense, int64_t query_tokens, int64_t query_start, int64_t seq_len, int64_t prompt_len) {
+  g_last_error[0] = '\0';
+  Geometry g;
+  if (plan_call(dense == 0, query_tokens, query_start, seq_len, dense == 0 ? prompt_len : seq_len, &g) != TM_OK) return -1;
+  return g.wide ? 1 : 0;
 }
 
 #ifdef TRIANGLEMIX_PLAN_OVERRIDE

@@ -1,5 +1,5 @@
-// Entry points of libtrianglemix.so for the torch adapter only: not part of
-// the public C ABI.  Same status codes and error text (tm_last_error) as there.
+// Entry points of libtrianglemix.so for the torch adapter and the tests: not
+// part of the public C ABI.  Same status codes and error text (tm_last_error) as there.
 #ifndef TRIANGLEMIX_INTERNAL_H
 #define TRIANGLEMIX_INTERNAL_H
 
@@ -18,6 +18,10 @@ int tmi_write_chunk_kv(const void* key, const void* value, void* key_cache, void
 // Those slots into slots[0 .. num_tokens - 1].
 int tmi_chunk_slots(const int32_t* block_table, int64_t table_cols, int64_t first_token, int64_t num_tokens,
                     int64_t* slots, void* stream);
+
+// Whether the kernel with 64 rows per wave runs this chunk (1 or 0; -1 for a
+// call the entry points refuse).  Arguments as tm_chunk_plan.
+int tmi_chunk_is_wide(int dense, int64_t query_tokens, int64_t query_start, int64_t seq_len, int64_t prompt_len);
 
 #ifdef __cplusplus
 }

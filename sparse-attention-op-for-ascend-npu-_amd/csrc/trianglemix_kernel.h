@@ -134,6 +134,11 @@ struct KernelParams {
 // range, items_per_head x 8 of four waves, two per CU).
 hipError_t launch_triangle_paged_attention(const KernelParams& p, bool sparse, int kv_parts, hipStream_t stream);
 
+// The same launch with 64 query rows per wave (trianglemix_wide.hip), for long
+// work items: the same items, splits, records and arrival words for each
+// kv_parts.
+hipError_t launch_wide_attention(const KernelParams& p, bool sparse, int kv_parts, hipStream_t stream);
+
 // Device address of this GPU's no-allocation scratch (kNoAllocScratchBytes,
 // 256-byte aligned), looked up once per device with the device current.
 hipError_t noalloc_scratch(void** ptr);

@@ -1,0 +1,113 @@
+"""The kernel with 64 query rows per wave (csrc/trianglemix_wide.hip), which runs plans whose items are long.
+
+Which kernel a chunk takes depends on its plan's longest item (csrc/trianglemix_capi.cpp long_items); both sides of
+each line are checked on the CPU.  On the GPU every row of chunks in each workgroup shape is compared with the fp32
+oracle, at the sizes where that kernel can go wrong: loop iterations at its line, tile counts that leave some KV
+parts one tile short, items of one, two and three iterations next to long ones, the 64-iteration blocks of the page
+table (one below, at and one above), rows that end inside a tile or a page, chunks that start off the 32-row and
+128-token grids, blocks that hold dense and sparse rows, one live row, split rows, and cache rows past the sequence
+that hold NaN.  Tolerances are the project's (max-abs 2e-2, mean-abs 2e-3, relative L2 2e-2 vs fp32).
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from test_gpu_any_length import _check_all_rows, _run
+from trianglemix import native
+from trianglemix.workload import make_cache, make_query
+
+
+def _is_wide(tq, qs, seq, prompt):
+    native.load_hip_library()
+    f = ctypes.CDLL(str(native.HIP_LIBRARY)).tmi_chunk_is_wide
+    f.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 4
+    return f(int(prompt is None), tq, qs, seq, prompt if prompt is not None else seq)
+
+
+# (query_start, query_tokens, prompt_len or None for the dense companion)
+LONG = [
+    # KV quarters
+    (512, 512, None),       # longest item 32 tiles: 8 iterations, the line; shortest 17 = 5 + 4 + 4 + 4
+    (479, 512, None),       # 31 tiles (8 + 8 + 8 + 7), rows off the 32-row grid
+    (488, 512, None),
+    (3584, 512, None),      # 32 iterations
+    (1477, 300, None),      # split in two, ragged
+    (8192, 100, 8292),      # dense tail split in four, four live rows in the last block
+    (8192, 100, None),
+    (8999, 1, None),        # one live row, split in eight
+    (29936, 64, None),
+    (4969, 31, 5000),       # one row block, split in five
+    (7680, 512, 8192),      # long dense-tail pieces beside 18-tile sparse items
+    (3584, 512, 4096),      # dense-tail rows unsplit beside sparse ones
+    # KV halves
+    (4096, 512, None),      # split in two
+    (7265, 512, None),      # up to 61 iterations, rows off the grids
+    (7680, 512, None),      # up to 64: one page-table block
+    (7788, 512, None),      # 65
+    (15872, 512, None),     # 128: two
+    (15988, 512, None),     # 129
+    (2048, 2048, None),     # unsplit, 33 .. 64 iterations
+    (15360, 1024, 16384),   # dense tail split in eight beside sparse items
+    # KV whole
+    (4096, 2048, 8320),     # sparse rows: 18 iterations
+    (1000, 1600, 9000),     # off the grids: 19
+    (2001, 1555, 70000),
+    (0, 2048, 8192),        # 1 .. 18 iterations: items shorter than the pipeline
+    (10297, 2048, None),    # 322 .. 386 iterations: six page-table blocks
+    (8192, 1024, None),     # split in two
+]
+SHORT = [(0, 512, 8192), (4096, 512, 8192), (0, 77, 77), (663, 37, None), (1000, 200, 1200), (8192, 1024, 32768),
+         (0, 2048, 2048), (6144, 2048, 8192)]
+
+
+def test_long_items_take_the_kernel_and_short_ones_do_not():
+    for qs, tq, prompt in LONG:
+        assert _is_wide(tq, qs, qs + tq, prompt) == 1, (qs, tq, prompt)
+    for qs, tq, prompt in SHORT:
+        assert _is_wide(tq, qs, qs + tq, prompt) == 0, (qs, tq, prompt)
+    assert _is_wide(512, 512, 1024, None) == 1 and _is_wide(512, 447, 959, None) == 1  # 32 and 30 tiles: 8 iterations
+    assert _is_wide(512, 384, 896, None) == 0  # 28 tiles: 7
+    assert _is_wide(512, 4000, 4608, 8192) == -1  # refused like the launch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qs,tq,prompt", LONG, ids=[f"{q}+{t}{'' if p else '_dense'}" for q, t, p in LONG])
+def test_long_items_match_oracle(gpu, qs, tq, prompt):
+    seq = qs + tq
+    print(f"long items qs={qs} tq={tq} prompt={prompt}", flush=True)
+    assert _is_wide(tq, qs, seq, prompt) == 1
+    k, v, bt = make_cache(seq, 40 + qs % 997, std=1.0)
+    # cache rows past the sequence must not matter
+    page, used = int(bt[0, (seq - 1) // 128]), (seq - 1) % 128 + 1
+    k[page, used:] = float("nan")
+    v[page, used:] = float("nan")
+    q = make_query(tq, 41 + tq % 991, std=1.0)
+    qd, kd, vd, btd = q.to(gpu), k.to(gpu), v.to(gpu), bt.to(gpu)
+    got = _run(gpu, qd, kd, vd, btd, qs, seq, prompt)
+    again = _run(gpu, qd, kd, vd, btd, qs, seq, prompt)
+    assert torch.equal(got, again)  # the merge order is fixed
+    kd[page, used:] = 0  # the blocked oracle multiplies whole pages
+    vd[page, used:] = 0
+    _check_all_rows(f"long items {qs}+{tq}", got, qd, kd, vd, btd, qs, seq, prompt)
+
+
+@pytest.mark.gpu
+def test_long_items_rescale(gpu):
+    """Scores that grow by far more than the lazy bound from tile to tile, and rows whose first tiles hold only
+    very low scores: every running max is replaced many times, in both heads of a wave."""
+    qs, tq = 512, 512
+    seq = qs + tq
+    k, v, bt = make_cache(seq, 77, std=1.0)
+    q = make_query(tq, 78, std=1.0)
+    flat = k.view(-1, 8, 128)
+    table = bt[0].tolist()
+    for t in range(seq):  # the key's length grows with its position, and shrinks again at the end
+        flat[table[t // 128] * 128 + t % 128] *= 0.05 * (t if t < 900 else 1900 - 2 * t)
+    qd, kd, vd, btd = q.to(gpu), k.to(gpu), v.to(gpu), bt.to(gpu)
+    assert _is_wide(tq, qs, seq, None) == 1
+    got = _run(gpu, qd, kd, vd, btd, qs, seq, None)
+    _check_all_rows("long items, growing scores", got, qd, kd, vd, btd, qs, seq, None)
