@@ -16,9 +16,10 @@ import ctypes
 import pytest
 import torch
 
+from oracle import attention as OA
 from test_gpu_any_length import _check_all_rows, _run
 from trianglemix import native
-from trianglemix.workload import make_cache, make_query
+from trianglemix.workload import SCALE, make_cache, make_query
 
 
 def _is_wide(tq, qs, seq, prompt):
@@ -43,6 +44,8 @@ LONG = [
     (4969, 31, 5000),       # one row block, split in five
     (7680, 512, 8192),      # long dense-tail pieces beside 18-tile sparse items
     (3584, 512, 4096),      # dense-tail rows unsplit beside sparse ones
+    (6000, 200, 6200),      # a block of sparse and dense-tail rows: its sparse rows skip most of its tiles
+    (4096, 400, 4496),
     # KV halves
     (4096, 512, None),      # split in two
     (7265, 512, None),      # up to 61 iterations, rows off the grids
@@ -52,6 +55,8 @@ LONG = [
     (15988, 512, None),     # 129
     (2048, 2048, None),     # unsplit, 33 .. 64 iterations
     (15360, 1024, 16384),   # dense tail split in eight beside sparse items
+    (10000, 300, 10300),    # a block of sparse and dense-tail rows, off the 32-row grid
+    (16384, 300, 16684),
     # KV whole
     (4096, 2048, 8320),     # sparse rows: 18 iterations
     (1000, 1600, 9000),     # off the grids: 19
@@ -59,6 +64,7 @@ LONG = [
     (0, 2048, 8192),        # 1 .. 18 iterations: items shorter than the pipeline
     (10297, 2048, None),    # 322 .. 386 iterations: six page-table blocks
     (8192, 1024, None),     # split in two
+    (0, 12300, 12300),      # a block of sparse and dense-tail rows, split; below it items of 1 to 19 tiles
 ]
 SHORT = [(0, 512, 8192), (4096, 512, 8192), (0, 77, 77), (663, 37, None), (1000, 200, 1200), (8192, 1024, 32768),
          (0, 2048, 2048), (6144, 2048, 8192)]
@@ -111,3 +117,39 @@ def test_long_items_rescale(gpu):
     assert _is_wide(tq, qs, seq, None) == 1
     got = _run(gpu, qd, kd, vd, btd, qs, seq, None)
     _check_all_rows("long items, growing scores", got, qd, kd, vd, btd, qs, seq, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qs,tq,prompt", [(6000, 200, 6200), (10000, 300, 10300), (0, 12300, 12300)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3e38], ids=["nan", "inf", "huge"])
+def test_sparse_rows_beside_dense_ones_ignore_the_keys_between(gpu, qs, tq, prompt, bad):
+    """Keys between the sink and the windows reach the dense-tail rows alone, also in the block that holds both
+    kinds of rows, whose sparse rows run through those keys' tiles and start anew behind them: whatever the keys
+    hold, every sparse row matches the oracle."""
+    seq = qs + tq
+    print(f"keys between qs={qs} tq={tq} prompt={prompt} bad={bad}", flush=True)
+    assert _is_wide(tq, qs, seq, prompt) == 1
+    tail = prompt - 128
+    assert (tail - qs) % 32 != 0  # dense-tail rows begin inside a block
+    k, v, bt = make_cache(seq, 51, std=1.0)
+    q = make_query(tq, 52, std=1.0)
+    # past the window of each row of that block, and for (0, ...) not past those of earlier rows, which see them
+    first_sparse = qs + (tail - qs) // 32 * 32
+    keys = [key for key in (40, 700, 2001, first_sparse - 512 - 40) if key >= 8]
+    reached = torch.zeros(tq, dtype=torch.bool)
+    rows = torch.arange(qs, seq)
+    at = [(int(bt[0, key // 128]), key % 128) for key in keys]
+    for key, (page, slot) in zip(keys, at):
+        k[page, slot] = bad
+        reached |= (rows >= key) & ((rows - key <= 512) | (rows < 521) | (rows >= tail))
+    qd, kd, vd, btd = q.to(gpu), k.to(gpu), v.to(gpu), bt.to(gpu)
+    got = _run(gpu, qd, kd, vd, btd, qs, seq, prompt)
+    for page, slot in at:
+        kd[page, slot] = 0
+    expected = OA.attention_torch_blocked(qd, kd, vd, btd, qs, seq, prompt, SCALE, max_scores=1 << 27)
+    free = (~reached).to(gpu)
+    block = torch.arange(first_sparse - qs, tail - qs, device=gpu)
+    assert free[block].all()
+    d = (got.float() - expected).abs()[free]
+    assert torch.isfinite(got[free].float()).all() and d.max().item() <= 2e-2 and d.mean().item() <= 2e-3
+    assert (got.float() - expected).abs()[block].mean().item() <= 2e-3
