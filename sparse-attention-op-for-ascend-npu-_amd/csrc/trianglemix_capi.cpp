@@ -321,39 +321,60 @@ ChunkPlan choose_plan(const std::vector<int>& row_tiles, bool sparse) {
 // loop iterations (tiles / KV parts), the eight-wave one otherwise.  The first
 // has the cheaper loop, the second the shorter start-up and merge, so the line
 // lies where the loop outweighs them, and higher where split rows merge in the
-// launch beside short sparse items.  Measured, us, eight-wave -> 64 rows per
-// wave, around each line:
-//  * KV quarters, nothing split or every row dense: 512 rows, longest item 4
-//    iterations 7.8 -> 7.9, 6 (split) 12.7 -> 12.7, 8 11.2 -> 10.7, 12 15.8 -> 14.7,
-//    32 39.0 -> 35.2;
-//  * KV quarters, split TriangleMix rows: 5 iterations 11.5 -> 13.0, 11 18.2 ->
-//    18.4 and 18.0 -> 19.1, 13 19.6 -> 21.1, 16 22.9 -> 19.8, 25.7 -> 23.7, 21
-//    29.8 -> 28.8;
+// launch: with KV quarters and halves if a TriangleMix chunk also has unsplit
+// rows, with KV whole always.  Measured, us, eight-wave -> 64 rows per wave,
+// around each line:
+//  * KV quarters, nothing split, or no row unsplit, or dense companion: 512 rows,
+//    longest item 4 iterations 7.8 -> 7.9, 6 (split) 12.7 -> 12.7, 8 11.2 -> 10.7,
+//    12 15.8 -> 14.7, 32 39.0 -> 35.2;
+//  * KV quarters, split and unsplit TriangleMix rows: 5 iterations 11.5 -> 13.0,
+//    11 18.2 -> 18.4 and 18.0 -> 19.1, 13 19.6 -> 21.1, 16 22.9 -> 19.8, 25.7 ->
+//    23.7, 21 29.8 -> 28.8;
 //  * KV halves: 9 iterations 13.6 -> 13.8, 14 (dense, split) 16.2 -> 15.8, 32
-//    40.0 -> 38.4, 64 104.5 -> 98.7; split TriangleMix rows: 11 16.9 -> 17.9,
-//    18 28.8 -> 29.7, 21 36.0 -> 35.0, 32 56.4 -> 55.5;
-//  * KV whole: 18 iterations 22.1 -> 21.6 and 20.2 -> 20.0, 576 557 -> 518;
-//    split, whose merge reads 66 KB per piece with two waves instead of four: 20
-//    iterations 43.1 -> 50.5, 64 101 -> 105, 144 147 -> 143, 256 308 -> 291.
+//    40.0 -> 38.4, 64 104.5 -> 98.7; split and unsplit TriangleMix rows: 11 16.9
+//    -> 17.9, 18 28.8 -> 29.7, 21 36.0 -> 35.0, 32 56.4 -> 55.5;
+//  * KV whole: 18 iterations 22.1 -> 21.6 and 20.2 -> 20.0, 576 557 -> 518 (it is
+//    planned only where the longest row has 17 tiles or more, so nothing lies
+//    below); split, whose merge reads 66 KB per piece with two waves instead of
+//    four: 20 iterations 43.1 -> 50.5, 64 101 -> 105, 144 147 -> 143, 256 308 -> 291.
+// Those KV-whole figures are of chunks whose items all run at once, or are long.
+// A KV-whole workgroup of two waves that has its CU to itself leaves half of the
+// SIMDs idle, one of four waves does not: with more items than slots, the short
+// ones left over at the end of a round cost more than the loop saves.  Then the
+// kernel is taken only if the items are long on average (mean tiles 40 211 -> 213,
+// 57 244 -> 235 and 313 -> 311, 64 142 -> 127, 96 218 -> 193) or one of them takes
+// nearly all of the simulated time (0.96-0.98 of it: prompts of 24576, 33000 and
+// 40960 tokens in one call 349 -> 327, 486 -> 459, 590 -> 547; 0.67 of it: 12300,
+// 16384 and 36000 tokens 157 -> 166, 202 -> 215, 450 -> 450).  2080 sparse rows
+// (65 items of 18 tiles) took 32.5 -> 39.0, 3072 35.6 -> 42.4, 8192 89 -> 95.
 struct LongItems {
-  int unsplit, split;  // fewest iterations: nothing split or every row dense; split TriangleMix rows
+  int unsplit, split;  // fewest iterations without and with merging split rows (see above)
 };
 constexpr LongItems kLongQuarters{8, 16};
 constexpr LongItems kLongHalves{14, 20};
-constexpr LongItems kLongWhole{16, 128};
+constexpr LongItems kLongWhole{1, 128};
+constexpr int kLongMeanTiles = 48;
+constexpr double kLongShare = 0.9;
 
 bool long_items(const std::vector<int>& row_tiles, const ChunkPlan& plan, bool sparse) {
   int64_t longest = 0;  // tiles of the longest item
-  bool split = false, short_rows = false;
+  int64_t items = 0, tiles = 0;
+  bool split = false, unsplit_rows = false;
   for (const int n : row_tiles) {
     const int64_t pieces = (n + plan.tiles_per_split - 1) / plan.tiles_per_split;
     longest = std::max(longest, (n + pieces - 1) / pieces);
+    items += pieces;
+    tiles += n;
     split = split || pieces > 1;
-    short_rows = short_rows || pieces == 1;
+    unsplit_rows = unsplit_rows || pieces == 1;
   }
   const LongItems& least = plan.kv_parts == 4 ? kLongQuarters : (plan.kv_parts == 2 ? kLongHalves : kLongWhole);
-  const bool merges = split && (plan.kv_parts == 1 || (sparse && short_rows));
-  return (longest + plan.kv_parts - 1) / plan.kv_parts >= (merges ? least.split : least.unsplit);
+  const bool merges = split && (plan.kv_parts == 1 || (sparse && unsplit_rows));
+  if ((longest + plan.kv_parts - 1) / plan.kv_parts < (merges ? least.split : least.unsplit)) return false;
+  if (plan.kv_parts != 1 || items <= kLargeWhole.slots || tiles >= kLongMeanTiles * items) return true;
+  return kLargeWhole.item_fixed + kLargeWhole.per_iteration * (double)longest >=
+         kLongShare * simulated_time(row_tiles, plan.tiles_per_split, kLargeWhole,
+                                     std::numeric_limits<double>::infinity());
 }
 
 // The choice depends only on the chunk geometry, which repeats for every layer

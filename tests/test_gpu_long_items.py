@@ -18,7 +18,7 @@ import torch
 
 from oracle import attention as OA
 from test_gpu_any_length import _check_all_rows, _run
-from trianglemix import native
+from trianglemix import cabi, native
 from trianglemix.workload import SCALE, make_cache, make_query
 
 
@@ -64,7 +64,7 @@ LONG = [
     (0, 2048, 8192),        # 1 .. 18 iterations: items shorter than the pipeline
     (10297, 2048, None),    # 322 .. 386 iterations: six page-table blocks
     (8192, 1024, None),     # split in two
-    (0, 12300, 12300),      # a block of sparse and dense-tail rows, split; below it items of 1 to 19 tiles
+    (64000, 2000, 66000),   # a block of sparse and dense-tail rows, split in twelve
 ]
 SHORT = [(0, 512, 8192), (4096, 512, 8192), (0, 77, 77), (663, 37, None), (1000, 200, 1200), (8192, 1024, 32768),
          (0, 2048, 2048), (6144, 2048, 8192)]
@@ -78,6 +78,15 @@ def test_long_items_take_the_kernel_and_short_ones_do_not():
     assert _is_wide(512, 512, 1024, None) == 1 and _is_wide(512, 447, 959, None) == 1  # 32 and 30 tiles: 8 iterations
     assert _is_wide(512, 384, 896, None) == 0  # 28 tiles: 7
     assert _is_wide(512, 4000, 4608, 8192) == -1  # refused like the launch
+    # KV whole, more items than the 64 slots: only if they are long on average, or one takes nearly all of the time
+    for tq, qs, prompt, wide in ((2048, 16384, 131072, 1), (2049, 16384, 131072, 0), (4096, 16384, 131072, 0),
+                                 (16384, 0, 131072, 0), (4096, 0, None, 1), (6000, 0, None, 1), (4096, 12288, None, 1),
+                                 (2048, 129024, 131072, 1), (6000, 60000, 66000, 1), (8192, 50000, 58192, 0),
+                                 (12300, 0, 12300, 0), (16384, 0, 16384, 0), (36000, 0, 36000, 0), (24576, 0, 24576, 1),
+                                 (33000, 0, 33000, 1), (40960, 0, 40960, 1)):
+        parts, _, items = cabi.chunk_plan(tq, qs, qs + tq, prompt)
+        assert parts == 1 and (items > 64 or tq == 2048)
+        assert _is_wide(tq, qs, qs + tq, prompt) == wide, (tq, qs, prompt)
 
 
 @pytest.mark.gpu
@@ -120,7 +129,7 @@ def test_long_items_rescale(gpu):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("qs,tq,prompt", [(6000, 200, 6200), (10000, 300, 10300), (0, 12300, 12300)])
+@pytest.mark.parametrize("qs,tq,prompt", [(6000, 200, 6200), (10000, 300, 10300), (64000, 2000, 66000)])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3e38], ids=["nan", "inf", "huge"])
 def test_sparse_rows_beside_dense_ones_ignore_the_keys_between(gpu, qs, tq, prompt, bad):
     """Keys between the sink and the windows reach the dense-tail rows alone, also in the block that holds both
@@ -133,7 +142,6 @@ def test_sparse_rows_beside_dense_ones_ignore_the_keys_between(gpu, qs, tq, prom
     assert (tail - qs) % 32 != 0  # dense-tail rows begin inside a block
     k, v, bt = make_cache(seq, 51, std=1.0)
     q = make_query(tq, 52, std=1.0)
-    # past the window of each row of that block, and for (0, ...) not past those of earlier rows, which see them
     first_sparse = qs + (tail - qs) // 32 * 32
     keys = [key for key in (40, 700, 2001, first_sparse - 512 - 40) if key >= 8]
     reached = torch.zeros(tq, dtype=torch.bool)
