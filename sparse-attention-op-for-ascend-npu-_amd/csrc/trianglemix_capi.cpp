@@ -353,6 +353,10 @@ struct LongItems {
 constexpr LongItems kLongQuarters{8, 16};
 constexpr LongItems kLongHalves{14, 20};
 constexpr LongItems kLongWhole{1, 128};
+// The eight-wave kernel's page table of a KV quarters or halves item has one block.
+static_assert(std::max(kLongQuarters.split, kLongQuarters.unsplit) * 4 <= tmx::kTableTiles + 4 &&
+                  std::max(kLongHalves.split, kLongHalves.unsplit) * 2 <= tmx::kTableTiles + 2,
+              "longer quarters and halves items run in the 64-row kernel");
 constexpr int kLongMeanTiles = 48;
 constexpr double kLongShare = 0.9;
 

@@ -53,9 +53,11 @@ static_assert(kMaxSplitItems < (1 << kEpochShift), "an arrival count fits below 
 // Split-KV scratch held per GPU for the no-allocation entry point (counter
 // block + partials): the largest workspace of any call.
 constexpr int64_t kNoAllocScratchBytes = kMaxWorkspaceBytes;
-// A work item may hold any number of tiles: the kernel keeps the page numbers
-// of 128 of them in two 64-lane registers and refills the one it has used up
-// while the other serves, 64 tiles at a time.
+// A kernel holds the page numbers of an item's tiles in 64-lane registers, a
+// block of 64 tiles each (64 per KV part in the 64-row kernel), and refills a
+// register once its block is used up: an item may hold any number of tiles.  The
+// eight-wave kernel's KV quarters and halves have one block and no refill; longer
+// items of theirs always run in the 64-row kernel.
 constexpr int kTableTiles = 64;
 // Most cache pages a launch accepts: the kernel addresses a key row of one KV
 // head by a 32-bit row index (page * 128 + slot) * 8 + head.  2^22 pages of
@@ -131,7 +133,8 @@ struct KernelParams {
 // workgroup shape: 4 (two query heads x KV quarters, items_per_head x 16
 // workgroups of eight waves), 2 (the four heads of the GQA group x KV halves,
 // items_per_head x 8 of eight waves) or 1 (the four heads x the whole KV
-// range, items_per_head x 8 of four waves, two per CU).
+// range, items_per_head x 8 of four waves, two per CU).  With 4 and 2 an item
+// holds at most kTableTiles tiles.
 hipError_t launch_triangle_paged_attention(const KernelParams& p, bool sparse, int kv_parts, hipStream_t stream);
 
 // The same launch with 64 query rows per wave (trianglemix_wide.hip), for long

@@ -22,9 +22,11 @@
 // of each of two KV-whole workgroups) let one wave's softmax run while the
 // other's MFMAs occupy the matrix core.
 // The KV tiles of a row block are cut into splits of at most
-// `tiles_per_split` tiles (host-chosen for load balance: at least 768 keys,
-// no upper bound -- an item of any length runs in one workgroup), so only
-// long dense rows split.  A row block with one
+// `tiles_per_split` tiles (host-chosen for load balance: at least 512 keys, no
+// upper bound), so only long dense rows split.  Long items run in the kernel
+// with 64 rows per wave (trianglemix_wide.hip; long_items in
+// trianglemix_capi.cpp draws the line): an item here has at most kTableTiles
+// tiles with KV quarters and halves, any number with KV whole.  A row block with one
 // split writes its output directly; otherwise every split writes an fp32
 // partial (O, row max, row sum) to the workspace and counts its arrival, and
 // the workgroup that arrives last merges all partials in split order
@@ -154,6 +156,11 @@ struct Shape {
   static constexpr int kWavesPerTile = kDmaPerTile / kDmaPerWave;   // waves sharing one tile's DMA
   static constexpr int kOwned = (kHeadDim / 32) / P;    // 32-wide d-blocks a wave keeps in the merge
   static constexpr int kQBlocksPerWave = 8 * kHeads / kWaves;  // 1 KB blocks of Q each wave DMAs
+  // Items of more than kTableTiles tiles: KV whole alone.  Without the second
+  // table, its page loads and the refill the other shapes' start-up is 300
+  // instructions shorter: a 77-row prompt 5.60 -> 5.46 us, the last 512 rows of
+  // 2869 19.6 -> 19.2, 512 sparse rows 9.85 -> 9.71.
+  static constexpr bool kLongItems = P == 1;
   static_assert((P == 4 || P == 2 || P == 1) && kHeads * P == kWaves && kHeads <= kGroup,
                 "supported shapes: 4 x 2, 2 x 4 and 1 x 4");
 };
@@ -276,11 +283,11 @@ triangle_paged_attention_kernel(const int32_t* block_table, const __bf16* query,
     const int slot = dma_t == 0 ? k_slot(row, lane & 15) : v_slot(row, lane & 15);
     dma_voff[j] = (unsigned)(row * kKvHeads * kRowBytes + 16 * slot);
   }
-  // DMA source of the item's tiles, 64 at a time: table block b (tiles 64b ..
-  // 64b + 63) lives in row_lo when b is even and in row_hi when b is odd,
-  // tile 64b + i in lane i.  The prologue fills blocks 0 and 1; an item of
-  // more than 128 tiles refills a register in the loop once its block has
-  // been issued (see refill below).  The value is the
+  // DMA source of the item's tiles, tile i in lane i of row_lo.  KV whole, whose
+  // items may be longer, holds them 64 at a time: table block b (tiles 64b ..
+  // 64b + 63) lives in row_lo when b is even and in row_hi when b is odd.  Its
+  // prologue fills blocks 0 and 1; an item of more than 128 tiles refills a
+  // register in the loop once its block has been issued (see refill below).  The value is the
   // cache row index of the tile's first key row of this KV head (its byte
   // offset / 256, below 2^32 as the host caps the cache at kMaxPages pages);
   // bytes_lo / bytes_hi hold the tile's valid byte count (rows cut at seq_len,
@@ -302,11 +309,11 @@ triangle_paged_attention_kernel(const int32_t* block_table, const __bf16* query,
     return __builtin_amdgcn_raw_buffer_load_b32(bt_rsrc, off, 0, 0);
   };
   const int phys_lo = lane_page(lane);
-  const int phys_hi = lane_page(kTableTiles + lane);
+  const int phys_hi = S::kLongItems ? lane_page(kTableTiles + lane) : 0;
   // Table block 2, for an item of more than 128 tiles (for a shorter one the
   // offset is out of range: the load returns 0 and touches no memory); the
   // loop turns it into rows when block 0 is used up (refill below).
-  int refill_phys = lane_page(2 * kTableTiles + lane);
+  int refill_phys = S::kLongItems ? lane_page(2 * kTableTiles + lane) : 0;
   // ---- Q: the workgroup's H heads x 32 rows (8 KB per head), DMA'd once into LDS ----
   // (each of the P part waves of a head needs all of it; loading it per wave
   // would multiply the start-up traffic through the CU).  Wave w loads the B =
@@ -338,9 +345,9 @@ triangle_paged_attention_kernel(const int32_t* block_table, const __bf16* query,
     return valid_rows > 0 ? (valid_rows - 1) * kKvHeads * kRowBytes + kRowBytes : 0;
   };
   unsigned row_lo = lane_row(lane, phys_lo);
-  unsigned row_hi = lane_row(kTableTiles + lane, phys_hi);
+  unsigned row_hi = S::kLongItems ? lane_row(kTableTiles + lane, phys_hi) : 0;
   int bytes_lo = lane_bytes(lane);
-  int bytes_hi = lane_bytes(kTableTiles + lane);
+  int bytes_hi = S::kLongItems ? lane_bytes(kTableTiles + lane) : 0;
   // The tile tables are complete here, before any tile DMA: left to itself the
   // compiler sinks the part it needs only for tiles 64-127 into the loop's
   // preheader, and the wait for its block-table load there would also wait
@@ -353,7 +360,7 @@ triangle_paged_attention_kernel(const int32_t* block_table, const __bf16* query,
   // empty range (its loads return zeros).
   auto tile_rsrc = [&](int ti, int t) {
     const unsigned u = (unsigned)ti;  // ti >= 0
-    const bool odd = ((u / kTableTiles) & 1) != 0;
+    const bool odd = S::kLongItems && ((u / kTableTiles) & 1) != 0;
     const unsigned row = __builtin_amdgcn_readlane(odd ? row_hi : row_lo, u % kTableTiles);
     const int bytes = ti < num_tiles ? __builtin_amdgcn_readlane(odd ? bytes_hi : bytes_lo, u % kTableTiles) : 0;
     const char* cache = reinterpret_cast<const char*>(t == 0 ? p.key_cache : p.value_cache);
@@ -496,7 +503,7 @@ triangle_paged_attention_kernel(const int32_t* block_table, const __bf16* query,
   m_run = m_tile;
   TM_PHASE(3);
 
-  // Table refill for items of more than 128 tiles.  Table block nb >= 2
+  // Table refill for items of more than 128 tiles (KV whole).  Table block nb >= 2
   // takes the register of block nb - 2.  The DMA of iteration it reaches
   // tile P (it + 2) + P - 1 (K) and P (it + 1) + P - 1 (V), so block nb - 2
   // is read for the last time in iteration 64 (nb - 1) / P - 2 and block nb
@@ -506,10 +513,10 @@ triangle_paged_attention_kernel(const int32_t* block_table, const __bf16* query,
   // and waited for by every iteration's wait for the wave's DMA since)
   // become rows and byte counts, and block nb + 1's page loads are issued.
   // One scalar compare per iteration; the refill itself is out of line.
-  int refill_it = num_tiles > 2 * kTableTiles ? kTableTiles / P - 1 : __INT_MAX__;
+  int refill_it = S::kLongItems && num_tiles > 2 * kTableTiles ? kTableTiles / P - 1 : __INT_MAX__;
   int refill_block = 2;
   auto refill = [&](int it) {
-    if (__builtin_expect(it == refill_it, 0)) {
+    if (S::kLongItems && __builtin_expect(it == refill_it, 0)) {
       const int ti = kTableTiles * refill_block + lane;
       const unsigned row = lane_row(ti, refill_phys);
       const int bytes = lane_bytes(ti);

@@ -12,7 +12,9 @@ that hold NaN.  Tolerances are the project's (max-abs 2e-2, mean-abs 2e-3, relat
 from __future__ import annotations
 
 import ctypes
+import random
 
+import plan_sweep
 import pytest
 import torch
 
@@ -87,6 +89,24 @@ def test_long_items_take_the_kernel_and_short_ones_do_not():
         parts, _, items = cabi.chunk_plan(tq, qs, qs + tq, prompt)
         assert parts == 1 and (items > 64 or tq == 2048)
         assert _is_wide(tq, qs, qs + tq, prompt) == wide, (tq, qs, prompt)
+
+
+def test_items_of_the_eight_wave_kernel_fit_its_page_table():
+    """With KV quarters and halves it holds one block of 64 tiles: any longer item runs in the 64-row kernel."""
+    rng = random.Random(7)
+    seen = {4: 0, 2: 0}
+    for _ in range(4000):
+        tq = round(2 ** rng.uniform(0, 11))
+        qs = rng.choice([0, round(2 ** rng.uniform(0, 16))])
+        prompt = rng.choice([None, qs + tq, qs + tq + rng.randrange(4096)])
+        parts, per_item, _ = cabi.chunk_plan(tq, qs, qs + tq, prompt)
+        if parts == 1 or _is_wide(tq, qs, qs + tq, prompt):
+            continue
+        tiles = plan_sweep.row_tiles(qs, tq, qs + tq, prompt or 0)
+        longest = max(-(-n // -(-n // per_item)) for n in tiles)
+        assert longest <= 64, (qs, tq, prompt)
+        seen[parts] = max(seen[parts], longest)
+    assert seen[4] > 50 and seen[2] > 30, seen  # near the lines: 60 and 38
 
 
 @pytest.mark.gpu
