@@ -19,6 +19,35 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
+// Phase clocks (diagnostic builds only, -DTRIANGLEMIX_PHASE_CLOCKS): lane 0 of
+// every wave stores the 100 MHz s_memrealtime clock at the TM_PHASE(slot)
+// points of the kernels, one 64-bit slot per (workgroup, wave, phase), for grids
+// of up to kPhaseClockWorkgroups workgroups.  Slots, the same in both kernels:
+//   0 entry, 1 page tables complete, 2 Q landed, 3 scores of the first tile done,
+//   4 + i iteration i opened (i < 8), 12 loop done, 13 KV parts merged,
+//   14 output stored (nothing split); of a split row block: 16 partials stored,
+//   17 arrival counted, 18 first batch of pieces merged, 19 all merged, 15 output
+//   stored.
+// Each source file has an array of its own; a launch fills that of its kernel
+// and the read-back joins them.  The product library is built without.
+#ifdef TRIANGLEMIX_PHASE_CLOCKS
+constexpr int kMaxWaves = 8;  // waves of the largest workgroup shape
+constexpr int kPhaseClockWorkgroups = 4096;
+constexpr int kPhaseClockSlots = 32;
+static __device__ unsigned long long phase_clocks[kPhaseClockWorkgroups * kMaxWaves * kPhaseClockSlots];
+hipError_t wide_phase_clocks(void** ptr);  // the array of trianglemix_wide.hip
+#define TM_PHASE(slot)                                                                                   \
+  do {                                                                                                   \
+    const unsigned long long tm_clock_ = __builtin_amdgcn_s_memrealtime();                               \
+    if ((threadIdx.x & 63) == 0 && blockIdx.x < kPhaseClockWorkgroups)                                   \
+      phase_clocks[(blockIdx.x * kMaxWaves + (threadIdx.x >> 6)) * kPhaseClockSlots + (slot)] = tm_clock_; \
+  } while (0)
+#else
+#define TM_PHASE(slot) \
+  do {                 \
+  } while (0)
+#endif
+
 #define TM_LDS(p) ((__attribute__((address_space(3))) void*)(p))
 
 constexpr int kRowBytes = kHeadDim * 2;          // 256 B: one key row

@@ -107,34 +107,15 @@
 #include <stdint.h>
 
 #include <mutex>
+#ifdef TRIANGLEMIX_PHASE_CLOCKS
+#include <vector>
+#endif
 
 #include "trianglemix_device.h"
 #include "trianglemix_kernel.h"
 
 namespace tmx {
 
-constexpr int kMaxWaves = 8;  // waves of the largest workgroup shape
-
-// Phase clocks (diagnostic builds only, -DTRIANGLEMIX_PHASE_CLOCKS): lane 0 of
-// every wave stores the 100 MHz s_memrealtime clock at the TM_PHASE(slot)
-// points below, one 64-bit slot per (workgroup, wave, phase),
-// for grids of up to kPhaseClockWorkgroups workgroups.  The product library
-// is built without them.
-#ifdef TRIANGLEMIX_PHASE_CLOCKS
-constexpr int kPhaseClockWorkgroups = 4096;
-constexpr int kPhaseClockSlots = 32;
-__device__ unsigned long long phase_clocks[kPhaseClockWorkgroups * kMaxWaves * kPhaseClockSlots];
-#define TM_PHASE(slot)                                                                                   \
-  do {                                                                                                   \
-    const unsigned long long tm_clock_ = __builtin_amdgcn_s_memrealtime();                               \
-    if ((threadIdx.x & 63) == 0 && blockIdx.x < kPhaseClockWorkgroups)                                   \
-      phase_clocks[(blockIdx.x * kMaxWaves + (threadIdx.x >> 6)) * kPhaseClockSlots + (slot)] = tm_clock_; \
-  } while (0)
-#else
-#define TM_PHASE(slot) \
-  do {                 \
-  } while (0)
-#endif
 // Workgroup shape: the waves are kParts KV parts x kHeads query heads.
 // P = 4 (two heads, KV quarters) puts a 512-token chunk's 16 row blocks on
 // 256 workgroups; P = 2 (all four heads of the GQA group, KV halves) loads
@@ -1052,15 +1033,28 @@ hipError_t noalloc_scratch(void** ptr) {
 
 #ifdef TRIANGLEMIX_PHASE_CLOCKS
 // Diagnostic exports of the phase-clock build: copy the clock slots to the
-// host, or clear them (before the launch to be read).
+// host (a slot is zero in the array of the kernel that did not run), or clear
+// them (before the launch to be read).
 extern "C" int tm_phase_clocks_read(void* host, int64_t bytes) {
   if (bytes < 0 || bytes > (int64_t)sizeof(phase_clocks)) return (int)hipErrorInvalidValue;
-  return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(phase_clocks), (size_t)bytes, 0, hipMemcpyDeviceToHost);
+  hipError_t err = hipMemcpyFromSymbol(host, HIP_SYMBOL(phase_clocks), (size_t)bytes, 0, hipMemcpyDeviceToHost);
+  if (err != hipSuccess) return (int)err;
+  void* address = nullptr;
+  err = wide_phase_clocks(&address);
+  if (err != hipSuccess) return (int)err;
+  std::vector<char> wide((size_t)bytes);
+  err = hipMemcpy(wide.data(), address, (size_t)bytes, hipMemcpyDeviceToHost);
+  for (size_t i = 0; i < wide.size(); ++i) static_cast<char*>(host)[i] |= wide[i];
+  return (int)err;
 }
 
 extern "C" int tm_phase_clocks_clear(void) {
   void* address = nullptr;
   hipError_t err = hipGetSymbolAddress(&address, HIP_SYMBOL(phase_clocks));
+  if (err != hipSuccess) return (int)err;
+  err = hipMemset(address, 0, sizeof(phase_clocks));
+  if (err != hipSuccess) return (int)err;
+  err = wide_phase_clocks(&address);
   if (err != hipSuccess) return (int)err;
   err = hipMemset(address, 0, sizeof(phase_clocks));
   if (err != hipSuccess) return (int)err;

@@ -105,6 +105,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
   const int lane = tid & 63;
   const int n = lane & 31;
   const int half = lane >> 5;
+  TM_PHASE(0);
 
   const int sparse_begin = kSparse ? pa.sparse_begin : 0;
   const int sparse_end = kSparse ? pa.sparse_end : 0;
@@ -237,6 +238,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     tab_mask = lane_mask(j - kMaskLag);
   };
   fill_tables(lane, phys0, vphys0);
+  TM_PHASE(1);
   auto read_rsrc = [&](unsigned w0, unsigned w1, int bytes, int i) TM_INLINE {
     const uint64_t at = (uint64_t)(unsigned)__builtin_amdgcn_readlane(w0, i) |
                         ((uint64_t)(unsigned)__builtin_amdgcn_readlane(w1, i) << 32);
@@ -319,6 +321,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     wait_dma_but<2 * S::kDma>();
   }
   __builtin_amdgcn_s_barrier();
+  TM_PHASE(2);
   bf16x8_t q_a[kHeadDim / 16], q_b[kHeadDim / 16];
   auto read_q = [&](bf16x8_t* qr, int head) TM_INLINE {
     const unsigned qb = (unsigned)(size_t)TM_LDS(q_lds + head * kRowBlock * kRowBytes) - (unsigned)tile_off;
@@ -478,6 +481,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
       s_a = mfma(kf[c], q_a[c], c == 0 ? f32x16_t{} : s_a);
       __builtin_amdgcn_sched_barrier(0);
     }
+    TM_PHASE(3);
     const __amdgpu_buffer_rsrc_t v2 = tile_rsrc(2, 1), k3 = tile_rsrc(3, 0);
     window(Yes{}, No{}, Yes{}, s_b, q_b, s_a, mask0, p_a, m_a, thr_a, l_a, o_a, [&](int st) TM_INLINE {
       // K(0) has been read: its last operand was waited for by the first QK^T
@@ -522,6 +526,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
   // kw: K slot of it + 1 (shared tiles: takes K of it + 1 + NS); vw: V slot of
   // it (takes V of it + NS); vr: V slot of it + 1.
   auto iteration = [&](int it, char* kr, char* kw, char* vw, char* vr) TM_INLINE {
+    if (it < 8) TM_PHASE(4 + it);
     const int kj = kPairs == 1 ? it + 2 + NS : it + 1 + NS;
     if (__builtin_expect((kj & (kTableTiles - 1)) == 0, 0)) {
       fill_tables(kj + lane, next_phys, next_vphys);
@@ -604,6 +609,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
   // The last two tiles: no QK^T follows the last one's.
   wait_dma();
   if (iters > 1) {
+    if (it < 8) TM_PHASE(4 + it);
     const int mask0 = __builtin_amdgcn_readfirstlane(lane_mask(iters - 1));
     window(Yes{}, Yes{}, No{}, s_b, q_b, s_a, mask0, p_a, m_a, thr_a, l_a, o_a, [&](int st) {
       if (kPairs == 2 && st == 2) __builtin_amdgcn_s_barrier();  // V of the last tile landed
@@ -629,6 +635,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     }
   }
 
+  TM_PHASE(12);
   // ---- merge the P KV parts through LDS ----
   // Part kq keeps d-blocks kq * O .. + O - 1 of both heads.
   constexpr int O = S::kOwned;
@@ -758,11 +765,13 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
   // Stage: q_lds, last read in the prologue (P = 2: by the merge above, which
   // must end first).
   char* const stage = q_lds;
+  TM_PHASE(13);
   if (nsplit == 1) {
     if constexpr (P == 2) __syncthreads();
     stage_rows(keep_a, l_a, 2 * pr, stage);
     stage_rows(keep_b, l_b, 2 * pr + 1, stage);
     store_stage(stage);
+    TM_PHASE(14);
     return;
   }
 
@@ -799,6 +808,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(l_b), rec, so + 256 + kStatL * 4, 0, kCpolAgent);
   }
   wait_dma();
+  TM_PHASE(16);
   __syncthreads();
   // the merge's reads of k_lds0 ended before the barrier above
   volatile int* s_last = reinterpret_cast<volatile int*>(k_lds0);
@@ -807,6 +817,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     *s_last = (int)(count_arrival(ctr, p.epoch) == (unsigned long long)nsplit);
   }
   __syncthreads();
+  TM_PHASE(17);
   if (!*s_last) return;
   if (tid == 0) __hip_atomic_store(ctr, p.epoch << kEpochShift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
@@ -879,7 +890,9 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
         }
         mt[h] = mu;
       }
+      if (s0 == 0) TM_PHASE(18);
     }
+    TM_PHASE(19);
     stage_rows(acc[0], lt[0], 2 * pr, stage);
     stage_rows(acc[1], lt[1], 2 * pr + 1, stage);
   } else {
@@ -925,12 +938,15 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
             }
           }
           mt = mu;
+          if (h == 0 && o == 0 && s0 == 0) TM_PHASE(18);
         }
         stage_block(acc, inverse(lt), 2 * pr + h, kq * O + o, stage);
       }
     }
+    TM_PHASE(19);
   }
   store_stage(stage);
+  TM_PHASE(15);
 }
 
 template <bool kSparse, int P>
@@ -944,6 +960,10 @@ hipError_t launch(const KernelParams& p, hipStream_t stream) {
 }
 
 }  // namespace
+
+#ifdef TRIANGLEMIX_PHASE_CLOCKS
+hipError_t wide_phase_clocks(void** ptr) { return hipGetSymbolAddress(ptr, HIP_SYMBOL(phase_clocks)); }
+#endif
 
 hipError_t launch_wide_attention(const KernelParams& p, bool sparse, int kv_parts, hipStream_t stream) {
   if (kv_parts == 1) return sparse ? launch<true, 1>(p, stream) : launch<false, 1>(p, stream);

@@ -89,6 +89,14 @@ def test_product_library_has_no_phase_clocks():
     assert mod.PHASE_CLOCK_LIB.name == "libtrianglemix_phase_clocks.so" and mod.PHASE_CLOCK_LIB != native.HIP_LIBRARY
 
 
+def test_both_attention_kernels_have_every_phase_clock():
+    """A chunk runs in either kernel: the diagnostic build must tell its phases in both."""
+    csrc = native.PKG_DIR.parent / "csrc"
+    slots = [set(re.findall(r"TM_PHASE\(([^)]+)\);", (csrc / f).read_text()))
+             for f in ("trianglemix_kernel.hip", "trianglemix_wide.hip")]
+    assert slots[0] == slots[1] and len(slots[0]) == 13, slots
+
+
 def test_product_library_has_no_plan_override():
     """Forcing the launch plan is compiled only into the sweep's diagnostic build (build.py --plan-override,
     its own file name)."""
