@@ -77,6 +77,14 @@ __device__ __forceinline__ void wait_dma_but() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// All but the last N (< 16) LDS reads of this wave have returned (lgkmcnt, bits
+// 11:8; LDS operations of a wave return in order).
+template <int N>
+__device__ __forceinline__ void wait_lds_but() {
+  static_assert(N >= 0 && N < 16, "lgkmcnt field");
+  __builtin_amdgcn_s_waitcnt(0xC07F | (N << 8));
+}
+
 __device__ __forceinline__ int k_slot(int row, int chunk) { return chunk ^ (row & 15); }
 __device__ __forceinline__ int v_slot(int row, int chunk) { return chunk ^ ((row & 3) << 2); }
 
@@ -162,15 +170,18 @@ __device__ __forceinline__ float half_sum(float x) {
 // first 32-lane half (the second half adds 4).
 __device__ __forceinline__ constexpr int elem_key(int v) { return 8 * (v >> 2) + (v & 3); }
 
-// MFMA step c of S^T = K Q^T (dims 16c .. 16c+15): the K operand from LDS.
+// MFMA step c of S^T = K Q^T (dims 16c .. 16c+15): the K operand from LDS, by
+// kKOperandReads read instructions.
+constexpr int kKOperandReads = 1;
 __device__ __forceinline__ bf16x8_t k_operand(const char* kt, const int* k_off, int c) {
   return *reinterpret_cast<const bf16x8_t*>(kt + k_off[c]);
 }
 
 // MFMA step k of O^T += V^T P^T (k = 0..7: d-block m = k % 4, k-group j = k / 4
-// of 16 keys): the V^T operand, two transposed reads.  k-slot e of half h in
+// of 16 keys): the V^T operand, kVOperandReads transposed reads.  k-slot e of half h in
 // k-group j is key 16j + 8(e/4) + 4h + e%4 -- the keys of P's bf16 lane
 // vector pb[j].
+constexpr int kVOperandReads = 2;
 __device__ __forceinline__ bf16x8_t v_operand(const char* vt, const int* v_off, int k) {
   const char* a0 = vt + 16 * (k >> 2) * kRowBytes + v_off[k & 3];
   const i16x4_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(a0));

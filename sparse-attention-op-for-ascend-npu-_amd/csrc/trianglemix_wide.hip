@@ -72,7 +72,29 @@ struct Wide {
   static constexpr int kOwned = (kHeadDim / 32) / P;     // 32-wide d-blocks per head a wave keeps in the merge
   static constexpr int kQBlocksPerWave = 8 * kHeads / kWaves;  // 1 KB blocks of Q each wave DMAs
   static constexpr int kStages = P == 4 ? 2 : 3;         // K and V slots
+  static_assert(kDma * kPairs == kDmaPerTile && kQBlocksPerWave * kWaves == 8 * kHeads, "the waves load whole tiles and Q");
+  static_assert((P == 1 ? 2 : 1) * (2 * kStages * kSlotBytes + kHeads * kRowBlock * kRowBytes) <= 160 * 1024,
+                "the workgroups of a CU (P = 1: two) fit its LDS");
 };
+
+// Wave-private tiles (P = 4): the operand that a step of a window reads, or -1.
+// Window 1 reads K, window 2 V; its last read falls behind the last step.
+constexpr int k_operand_at(int st) { return (st & 1) != 0 ? st >> 1 : -1; }
+constexpr int v_operand_at(int st) { return (st & 1) == 0 && st > 0 ? (st >> 1) - 1 : -1; }
+static_assert(k_operand_at(15) == 7 && v_operand_at(16) == 7, "a window reads eight operands");
+// From this step of a window on its DMA refills the slot that the window before
+// read; `but` counts the LDS reads issued since the last of those.
+constexpr int kRefillStep = 6;
+constexpr int k_reads_but() {
+  int n = 0;
+  for (int st = 0; st < kRefillStep; ++st) n += k_operand_at(st) >= 0 ? kKOperandReads : 0;
+  return n;
+}
+constexpr int v_reads_but() {
+  int n = 0;
+  for (int st = 0; st < kRefillStep; ++st) n += v_operand_at(st) >= 0 ? kVOperandReads : 0;
+  return n;
+}
 
 // Row max (log2 units) of a row that has met no attended key: finite, so that
 // exp2(-inf - max) = 0 without a test, and so low that any real max's rescale
@@ -506,11 +528,11 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     if (iters > 1) {
       window(Yes{}, No{}, Yes{}, s_a, q_a, s_b, mask0, p_b, m_b, thr_b, l_b, o_b, [&](int st) TM_INLINE {
         if (kPairs == 1) {
-          // K(1) has been read (two operands of V were read since)
-          if (st == 6) __builtin_amdgcn_s_waitcnt(0xC47F);
-          if (st >= 6 && st < 14) dma_k(k3, k_lds1, st - 6, dma_base);
+          // K(1) has been read
+          if (st == kRefillStep) wait_lds_but<v_reads_but()>();
+          if (st >= kRefillStep && st < kRefillStep + 8) dma_k(k3, k_lds1, st - kRefillStep, dma_base);
         }
-        if ((st & 1) == 0 && st > 0) read_v(v_lds0, (st >> 1) - 1);
+        if (v_operand_at(st) >= 0) read_v(v_lds0, v_operand_at(st));
       });
     } else {
       window(No{}, No{}, Yes{}, s_a, q_a, s_b, mask0, p_b, m_b, thr_b, l_b, o_b, [&](int st) TM_INLINE {
@@ -557,20 +579,20 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
           else dma_k(k_rsrc, kw, (st - 8) >> 1, dma_at);
         }
       } else {
-        // V(it) has been read (K's first three reads were issued since)
-        if (st == 6) __builtin_amdgcn_s_waitcnt(0xC37F);
-        if (st & 1) read_k(kr, st >> 1);
-        if (st >= 6 && st < 14) dma_v(v_rsrc, vw, st - 6, dma_at);
+        // V(it) has been read
+        if (st == kRefillStep) wait_lds_but<k_reads_but()>();
+        if (k_operand_at(st) >= 0) read_k(kr, k_operand_at(st));
+        if (st >= kRefillStep && st < kRefillStep + 8) dma_v(v_rsrc, vw, st - kRefillStep, dma_at);
       }
     });
     if (kPairs == 1) wait_dma_but<2 * kD>();  // V(it + 1) landed; behind it K(it + 3), V(it + 2)
     window(Yes{}, Yes{}, No{}, s_a, q_a, s_b, mask0, p_b, m_b, thr_b, l_b, o_b, [&](int st) {
       if (kPairs == 1) {
-        // K(it + 2) has been read (two operands of V were read since)
-        if (st == 6) __builtin_amdgcn_s_waitcnt(0xC47F);
-        if (st >= 6 && st < 14) dma_k(k_rsrc, kr, st - 6, dma_at);
+        // K(it + 2) has been read
+        if (st == kRefillStep) wait_lds_but<v_reads_but()>();
+        if (st >= kRefillStep && st < kRefillStep + 8) dma_k(k_rsrc, kr, st - kRefillStep, dma_at);
       }
-      if ((st & 1) == 0 && st > 0) read_v(vr, (st >> 1) - 1);
+      if (v_operand_at(st) >= 0) read_v(vr, v_operand_at(st));
     });
   };
   int it = 0;
@@ -617,7 +639,7 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     const int vs = (iters - 1) % NS;
     const char* vr = vs == 0 ? v_lds0 : (vs == 1 ? v_lds1 : v_lds2);
     window(No{}, Yes{}, No{}, s_a, q_a, s_b, mask0, p_b, m_b, thr_b, l_b, o_b, [&](int st) {
-      if ((st & 1) == 0 && st > 0) read_v(vr, (st >> 1) - 1);
+      if (v_operand_at(st) >= 0) read_v(vr, v_operand_at(st));
     });
   }
   if (kPairs == 2) {
@@ -654,6 +676,13 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
     // taken the barrier of the second-to-last iteration; an item of one
     // iteration had no such barrier.
     if (kPairs == 2 && num_iters == 1) __syncthreads();
+    constexpr int kStretch = 4 * 64 * 16, kStats = 4 * 64 * 4;
+    static_assert(P != 4 || (S::kWaves * kTileBytes == S::kSlotBytes && 2 * kStretch <= kTileBytes &&
+                             kStats <= kTileBytes && 4 - O == 3),
+                  "P = 4: a given block of both heads fits the wave's tile of each of three slots, the statistics the fourth's");
+    static_assert(P != 2 || (S::kWaves * kStretch <= S::kSlotBytes && S::kWaves * kStretch <= 16384 && 4 - O == 2 &&
+                             16384 + S::kWaves * kStats <= H * kRowBlock * kRowBytes),
+                  "P = 2: three K slots and half of q_lds hold the given blocks, the rest of q_lds the statistics");
     auto xo = [&](int g, int gi, int w) -> f32x4_t* {  // head g, gi-th given block, wave w
       if constexpr (P == 4) {
         char* base = gi == 0 ? k_lds0 : (gi == 1 ? k_lds1 : v_lds0);
@@ -729,6 +758,9 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
   constexpr int kChunksPerRow = kStageRow / 16;
   constexpr int kRowsPerStore = 64 / kChunksPerRow;
   constexpr int kStores = kRowBlock / (kRowsPerStore * S::kWaves);
+  static_assert(kRowsPerStore * kChunksPerRow == 64 && kStores * kRowsPerStore * S::kWaves == kRowBlock,
+                "the stores cover the row block");
+  static_assert(kRowBlock * kStageRow <= H * kRowBlock * kRowBytes, "the stage fits q_lds");
   auto stage_block = [&](const f32x16_t& blk, float inv, int head, int m, char* stage) TM_INLINE {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
