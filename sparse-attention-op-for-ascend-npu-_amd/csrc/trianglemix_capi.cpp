@@ -624,12 +624,12 @@ int launched(hipError_t err) {
   return fail(TM_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
 }
 
-// Checks of a paged KV write; index is the slot mapping or block table
-// (index_bytes long) the slots come from.  TM_OK with num_tokens == 0 means
+// Checks of a paged KV write; index, called index_name in messages, is the slot
+// mapping or block table (index_bytes long) the slots come from.  TM_OK with num_tokens == 0 means
 // nothing to write, whatever the pointers.
 int check_kv_write(const void* key, const void* value, const void* key_cache, const void* value_cache,
-                   const void* index, int64_t index_bytes, int64_t num_tokens, int64_t key_stride,
-                   int64_t value_stride, int64_t num_pages) {
+                   const void* index, const char* index_name, int64_t index_bytes, int64_t num_tokens,
+                   int64_t key_stride, int64_t value_stride, int64_t num_pages) {
   g_last_error[0] = '\0';
   if (num_tokens < 0 || num_tokens > tmx::kMaxPositions) {
     return fail(TM_ERR_INVALID_ARGUMENT, "key and value must be [num_tokens, 8, 128] with 0 <= num_tokens <= %lld",
@@ -644,7 +644,7 @@ int check_kv_write(const void* key, const void* value, const void* key_cache, co
   }
   if (num_tokens == 0) return TM_OK;
   if (!key || !value || !key_cache || !value_cache || !index) {
-    return fail(TM_ERR_INVALID_ARGUMENT, "key, value, key_cache, value_cache and slot_mapping must be non-null");
+    return fail(TM_ERR_INVALID_ARGUMENT, "key, value, key_cache, value_cache and %s must be non-null", index_name);
   }
   constexpr int64_t kRowElems = int64_t(tmx::kKvHeads) * tmx::kHeadDim;
   if (key_stride < kRowElems || value_stride < kRowElems || key_stride % 8 != 0 || value_stride % 8 != 0) {
@@ -665,7 +665,7 @@ int check_kv_write(const void* key, const void* value, const void* key_cache, co
   if (overlaps(r_kc, r_vc) || overlaps(r_kc, r_k) || overlaps(r_kc, r_v) || overlaps(r_kc, r_s) ||
       overlaps(r_vc, r_k) || overlaps(r_vc, r_v) || overlaps(r_vc, r_s)) {
     return fail(TM_ERR_INVALID_ARGUMENT,
-                "key_cache and value_cache must not overlap each other, key, value or slot_mapping");
+                "key_cache and value_cache must not overlap each other, key, value or %s", index_name);
   }
   return TM_OK;
 }
@@ -801,8 +801,8 @@ void tm_plan_override(int32_t kv_parts, int32_t tiles_per_split) {
 int tm_reshape_and_cache(const void* key, const void* value, void* key_cache, void* value_cache,
                          const int64_t* slot_mapping, int64_t num_tokens, int64_t key_stride, int64_t value_stride,
                          int64_t num_pages, void* stream) {
-  const int st = check_kv_write(key, value, key_cache, value_cache, slot_mapping, num_tokens * 8, num_tokens,
-                                key_stride, value_stride, num_pages);
+  const int st = check_kv_write(key, value, key_cache, value_cache, slot_mapping, "slot_mapping", num_tokens * 8,
+                                num_tokens, key_stride, value_stride, num_pages);
   if (st != TM_OK || num_tokens == 0) return st;  // 0 tokens: nothing to write, nothing enqueued
   return launched(tmx::launch_paged_kv_write(key, value, key_cache, value_cache, slot_mapping, num_tokens, key_stride,
                                              value_stride, num_pages, static_cast<hipStream_t>(stream)));
@@ -811,8 +811,8 @@ int tm_reshape_and_cache(const void* key, const void* value, void* key_cache, vo
 int tmi_write_chunk_kv(const void* key, const void* value, void* key_cache, void* value_cache,
                        const int32_t* block_table, int64_t table_cols, int64_t first_token, int64_t num_tokens,
                        int64_t key_stride, int64_t value_stride, int64_t num_pages, void* stream) {
-  int st = check_kv_write(key, value, key_cache, value_cache, block_table, table_cols * 4, num_tokens, key_stride,
-                          value_stride, num_pages);
+  int st = check_kv_write(key, value, key_cache, value_cache, block_table, "block_table", table_cols * 4, num_tokens,
+                          key_stride, value_stride, num_pages);
   if (st == TM_OK) st = check_chunk_table(table_cols, first_token, num_tokens);
   if (st != TM_OK || num_tokens == 0) return st;
   return launched(tmx::launch_chunk_kv_write(key, value, key_cache, value_cache, block_table, first_token, num_tokens,

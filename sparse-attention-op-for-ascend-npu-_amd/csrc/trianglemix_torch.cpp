@@ -205,13 +205,13 @@ at::Tensor& dense_paged_causal_attention_out(const at::Tensor& query, const at::
   return output;
 }
 
-// Checks of a paged KV write; `index` (the slot mapping or the block table)
-// lies on the same device.  key / value may be row-strided views (a slice of
+// Checks of a paged KV write; `index` (the slot mapping or the block table, as
+// index_name says) lies on the same device.  key / value may be row-strided views (a slice of
 // a fused QKV buffer); their [8, 128] part must be contiguous.
 void check_kv_write(const at::Tensor& key, const at::Tensor& value, const at::Tensor& key_cache,
-                    const at::Tensor& value_cache, const at::Tensor& index) {
+                    const at::Tensor& value_cache, const at::Tensor& index, const char* index_name) {
   TORCH_CHECK(key.is_cuda() && value.is_cuda() && key_cache.is_cuda() && value_cache.is_cuda() && index.is_cuda(),
-              "key, value, key_cache, value_cache and slot_mapping must be GPU tensors");
+              "key, value, key_cache, value_cache and ", index_name, " must be GPU tensors");
   TORCH_CHECK(key.device() == value.device() && key.device() == key_cache.device() &&
                   key.device() == value_cache.device() && key.device() == index.device(),
               "all inputs must be on the same GPU device");
@@ -241,7 +241,7 @@ void check_kv_shapes(const at::Tensor& key, const at::Tensor& value, const at::T
 // (negative = padding, skipped).
 void reshape_and_cache(const at::Tensor& key, const at::Tensor& value, at::Tensor& key_cache, at::Tensor& value_cache,
                        const at::Tensor& slot_mapping) {
-  check_kv_write(key, value, key_cache, value_cache, slot_mapping);
+  check_kv_write(key, value, key_cache, value_cache, slot_mapping, "slot_mapping");
   TORCH_CHECK(slot_mapping.scalar_type() == at::ScalarType::Long && slot_mapping.dim() == 1 &&
                   slot_mapping.is_contiguous(),
               "slot_mapping must be a contiguous INT64 [num_tokens] tensor");
@@ -284,7 +284,7 @@ at::Tensor chunk_slots(const at::Tensor& block_table, int64_t query_start, int64
 // reshape_and_cache of those tokens in one launch, without a slot mapping.
 void write_chunk_kv(const at::Tensor& key, const at::Tensor& value, at::Tensor& key_cache, at::Tensor& value_cache,
                     const at::Tensor& block_table, int64_t query_start) {
-  check_kv_write(key, value, key_cache, value_cache, block_table);
+  check_kv_write(key, value, key_cache, value_cache, block_table, "block_table");
   check_table(block_table);
   TORCH_CHECK(key.dim() == 3 && key.size(1) == 8 && key.size(2) == 128 && value.sizes() == key.sizes(),
               "key and value must be [num_tokens, 8, 128]");

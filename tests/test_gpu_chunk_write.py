@@ -6,6 +6,8 @@ table that the native path does not take, which must give the same slots.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -36,6 +38,24 @@ def test_forms_the_native_path_leaves_to_tensor_operations():
             rows = torch.zeros(n, 8, 128, dtype=torch.bfloat16)
             with pytest.raises(ValueError):
                 cache.write_chunk_kv(rows, rows, None, None, table, start)
+
+
+def test_messages_name_the_index_that_was_passed():
+    """The refusals of the C entry points: every check runs before any GPU call."""
+    lib = native.load_hip_library()
+    raw = ctypes.CDLL(str(native.HIP_LIBRARY))
+    p, i64 = ctypes.c_void_p, ctypes.c_int64
+    raw.tmi_write_chunk_kv.argtypes = [p] * 5 + [i64] * 6 + [p]
+    raw.tm_reshape_and_cache.argtypes = [p] * 5 + [i64] * 4 + [p]
+    page = 128 * 8 * 128 * 2
+    key, value, kc, vc = 1 << 20, 2 << 20, 3 << 20, (3 << 20) + page
+    for index, message in ((None, "must be non-null"), (kc, "must not overlap")):
+        assert raw.tmi_write_chunk_kv(key, value, kc, vc, index, 1, 0, 1, 1024, 1024, 1, None) == 1
+        error = lib.tm_last_error().decode()
+        assert message in error and "block_table" in error and "slot_mapping" not in error
+        assert raw.tm_reshape_and_cache(key, value, kc, vc, index, 1, 1024, 1024, 1, None) == 1
+        error = lib.tm_last_error().decode()
+        assert message in error and "slot_mapping" in error
 
 
 @pytest.mark.gpu
@@ -81,6 +101,8 @@ def test_chunk_write_refuses_what_the_mapped_write_refuses(gpu):
         cache.write_chunk_kv(rows[:, :4], rows[:, :4], kc, vc, table, 0)
     with pytest.raises(RuntimeError):
         cache.write_chunk_kv(rows, rows, kc, kc, table, 0)  # the caches overlap
+    with pytest.raises(RuntimeError, match="and block_table must be GPU tensors"):
+        torch.ops.trianglemix.write_chunk_kv(rows, rows, kc, vc, table.cpu(), 0)
     with pytest.raises(RuntimeError, match="lacks logical pages"):
         torch.ops.trianglemix.write_chunk_kv(rows, rows, kc, vc, table, 253)
     cache.write_chunk_kv(rows[:0], rows[:0], kc, vc, table, 256)  # nothing to write
