@@ -1,8 +1,9 @@
 """The kernel with 64 query rows per wave (csrc/trianglemix_wide.hip), which runs plans whose items are long.
 
-Which kernel a chunk takes depends on its plan's longest item (csrc/trianglemix_capi.cpp long_items); both sides of
-each line are checked on the CPU.  On the GPU every row of chunks in each workgroup shape is compared with the fp32
-oracle, at the sizes where that kernel can go wrong: loop iterations at its line, tile counts that leave some KV
+Which kernel a chunk takes depends on its plan's longest item (csrc/trianglemix_capi.cpp long_items); the plan, the
+iterations and the kernel of a chunk on either side of each line are checked on the CPU.  On the GPU every row of
+chunks in each workgroup shape is compared with the fp32 oracle, those on either side of each line among them, at
+the sizes where the 64-row kernel can go wrong: loop iterations at its line, tile counts that leave some KV
 parts one tile short, items of one, two and three iterations next to long ones, the 64-iteration blocks of the page
 table (one below, at and one above), rows that end inside a tile or a page, chunks that start off the 32-row and
 128-token grids, blocks that hold dense and sparse rows, one live row, split rows, and cache rows past the sequence
@@ -72,6 +73,36 @@ SHORT = [(0, 512, 8192), (4096, 512, 8192), (0, 77, 77), (663, 37, None), (1000,
          (0, 2048, 2048), (6144, 2048, 8192)]
 
 
+# One iteration below each line and at it: (query_start, query_tokens, prompt_len, KV parts, rows split, some split and
+# others not, iterations of the longest item, 64-row kernel).
+LINES = [
+    (864, 15, None, 4, False, False, 7, 0),
+    (949, 30, None, 4, False, False, 8, 1),
+    (6144, 2, 6224, 4, True, False, 7, 0),     # all rows split: the lower line
+    (7328, 2, 7330, 4, True, False, 8, 1),
+    (5312, 163, 5475, 4, True, True, 15, 0),   # split and unsplit rows: the higher one
+    (3795, 228, 4023, 4, True, True, 16, 1),
+    (190, 608, 798, 2, False, False, 13, 0),
+    (224, 614, 838, 2, False, False, 14, 1),
+    (342, 621, None, 2, True, True, 14, 1),    # of the dense companion: the lower line
+    (8117, 160, 8277, 2, True, True, 19, 0),
+    (8439, 160, 8599, 2, True, True, 20, 1),
+    (7052, 1024, None, 1, True, False, 127, 0),
+    (12000, 544, None, 1, True, False, 128, 1),
+]
+
+
+@pytest.mark.parametrize("qs,tq,prompt,parts,split,mixed,iterations,wide", LINES)
+def test_either_side_of_each_line(qs, tq, prompt, parts, split, mixed, iterations, wide):
+    plan_parts, per_item, _ = cabi.chunk_plan(tq, qs, qs + tq, prompt)
+    tiles = plan_sweep.row_tiles(qs, tq, qs + tq, prompt or 0)
+    pieces = plan_sweep.pieces(tiles, per_item)
+    longest = max(-(-n // k) for n, k in zip(tiles, pieces))
+    assert (plan_parts, max(pieces) > 1, max(pieces) > 1 and min(pieces) == 1, -(-longest // parts)) == (
+        parts, split, mixed, iterations)
+    assert _is_wide(tq, qs, qs + tq, prompt) == wide
+
+
 def test_long_items_take_the_kernel_and_short_ones_do_not():
     for qs, tq, prompt in LONG:
         assert _is_wide(tq, qs, qs + tq, prompt) == 1, (qs, tq, prompt)
@@ -109,12 +140,15 @@ def test_items_of_the_eight_wave_kernel_fit_its_page_table():
     assert seen[4] > 50 and seen[2] > 30, seen  # near the lines: 60 and 38
 
 
+ALL = [(*c, 1) for c in LONG] + [(*c[:3], c[-1]) for c in LINES]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("qs,tq,prompt", LONG, ids=[f"{q}+{t}{'' if p else '_dense'}" for q, t, p in LONG])
-def test_long_items_match_oracle(gpu, qs, tq, prompt):
+@pytest.mark.parametrize("qs,tq,prompt,wide", ALL, ids=[f"{q}+{t}{'' if p else '_dense'}" for q, t, p, _ in ALL])
+def test_long_items_match_oracle(gpu, qs, tq, prompt, wide):
     seq = qs + tq
     print(f"long items qs={qs} tq={tq} prompt={prompt}", flush=True)
-    assert _is_wide(tq, qs, seq, prompt) == 1
+    assert _is_wide(tq, qs, seq, prompt) == wide
     k, v, bt = make_cache(seq, 40 + qs % 997, std=1.0)
     # cache rows past the sequence must not matter
     page, used = int(bt[0, (seq - 1) // 128]), (seq - 1) % 128 + 1
@@ -146,6 +180,33 @@ def test_long_items_rescale(gpu):
     assert _is_wide(tq, qs, seq, None) == 1
     got = _run(gpu, qd, kd, vd, btd, qs, seq, None)
     _check_all_rows("long items, growing scores", got, qd, kd, vd, btd, qs, seq, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qs,tq,prompt,parts,split", [
+    (5669, 31, 5700, 4, True), (224, 614, 838, 2, False), (342, 621, None, 2, True),
+    (10297, 2048, None, 1, False), (12000, 544, None, 1, True)])
+def test_long_items_rescale_in_the_other_shapes(gpu, qs, tq, prompt, parts, split):
+    """The same with split KV quarters, halves and KV whole, split and not, whose waves share their tiles."""
+    seq = qs + tq
+    plan_parts, per_item, _ = cabi.chunk_plan(tq, qs, seq, prompt)
+    assert plan_parts == parts and ((seq + 31) // 32 > per_item) == split
+    k, v, bt = make_cache(seq, 77, std=1.0)
+    # One key takes nearly all of a row, so outputs are as large as V's entries (|v| < 6 of millions of N(0, 1)):
+    # bf16's rounding of the output (2^-6 for 4 <= |v| < 8) and of the probabilities (2^-9 |v|) come to 2.7e-2,
+    # and with V halved to 1.4e-2, below the 2e-2 asked for.
+    v *= 0.5
+    q = make_query(tq, 78, std=1.0)
+    # the key's length grows with its position up to 45 times, and shrinks again at the end
+    t, top = torch.arange(seq, dtype=torch.float32), seq * 0.88
+    length = 45.0 * torch.where(t < top, t, 2 * top - t) / top
+    for page in range((seq + 127) // 128):
+        n = min(128, seq - 128 * page)
+        k[int(bt[0, page]), :n] *= length[128 * page:128 * page + n].to(torch.bfloat16).view(-1, 1, 1)
+    qd, kd, vd, btd = q.to(gpu), k.to(gpu), v.to(gpu), bt.to(gpu)
+    assert _is_wide(tq, qs, seq, prompt) == 1
+    got = _run(gpu, qd, kd, vd, btd, qs, seq, prompt)
+    _check_all_rows("long items, growing scores", got, qd, kd, vd, btd, qs, seq, prompt)
 
 
 @pytest.mark.gpu
