@@ -88,6 +88,13 @@ int check_attributes(int64_t query_tokens, int64_t query_start, int64_t seq_len,
 // plan's time is its latest slot or split row block.  The candidate with the
 // shortest simulated time is taken (ties: the larger T, fewer partials).
 //
+// The costs are those of the eight-wave kernel, fitted when it ran every plan.
+// Plans with long items have since moved to the kernel with 64 rows per wave
+// (long_items below), which is chosen after the plan and not costed: 87 planned
+// chunks took 6,700 us in the eight-wave kernel and take 6,187 so, K and V from
+// HBM, but what other plans would take in the other kernel is not known, and the
+// times below are the eight-wave kernel's.
+//
 // Three regimes, with costs fitted on MI355X to sweeps of forced plans (every
 // candidate plan of each geometry timed as 20 launches, fastest of three
 // passes, HIP events): 87 TriangleMix and dense-companion chunks of 64 to

@@ -1,8 +1,9 @@
 // The attention kernel for long work items: 64 query rows per wave.
 //
-// Same operator, items, splits, tile schedule, LDS layout, masks and numerics
-// as triangle_paged_attention_kernel (trianglemix_kernel.hip); another shape
-// of wave.  There a wave owns 32 rows (one query head) and two waves share a
+// Same operator, items, splits, tiles, LDS layout and numerics as
+// triangle_paged_attention_kernel (trianglemix_kernel.hip), and the same masks
+// in the result (a block of sparse and dense rows takes its tiles in another
+// order); another shape of wave.  There a wave owns 32 rows (one query head) and two waves share a
 // SIMD; here it owns 64 (a pair of heads of the GQA group over the same 32
 // tokens) and has the SIMD, with up to 512 registers, to itself:
 //  * P = 4: four waves, one head pair x four KV parts, 16 workgroups per item;
@@ -410,8 +411,8 @@ wide_attention_kernel(const int32_t* block_table, const __bf16* query, int query
   // Half an iteration of the pipeline, 16 steps: the QK^T MFMAs of head y
   // (even steps) alternate with the PV MFMAs of head x's present tile (odd
   // steps) -- two independent chains -- while the VALU takes the row max and
-  // the exponentials of head x's next tile (scores s_x; its QK^T ended the window before) into p_x.  `mem` issues each step's LDS
-  // reads and DMA.  A tile's 16 probabilities per lane are summed by themselves and
+  // the exponentials of head x's next tile (scores s_x; its QK^T ended the
+  // window before) into p_x.  `mem` issues each step's LDS reads and DMA.  A tile's 16 probabilities per lane are summed by themselves and
   // added once to the running row sum, so that the row sum is rounded once per
   // tile against the whole sum, as in the eight-wave kernel, and not 16 times
   // (one dominant key and all others alike, 1024 tiles: the outputs were 2.8e-4

@@ -9,10 +9,13 @@ forward order over the plans, keeping each plan's fastest.  Inputs are seeded N(
 page table, generated on the GPU.  Geometries marked ``held_out`` were not used for the first fit, only
 to check it.
 
-Run on the GPU box from the repository root after ``python sparse-attention-op-for-ascend-npu-_amd/build.py
+The committed sweep was taken when the eight-wave kernel ran every plan.  A forced plan now runs in the
+kernel that the dispatch rule (``long_items``) picks for it, so a new sweep times plan and kernel together.
+
+Run on an MI355X from the repository root after ``python sparse-attention-op-for-ascend-npu-_amd/build.py
 --plan-override``:
 
-    python tests/plan_sweep.py --out gpurun_out/plan_sweep_mi355x.json
+    python tests/plan_sweep.py --out sweep.json
 """
 
 from __future__ import annotations
@@ -113,7 +116,7 @@ def candidates(rt: list[int]) -> list[tuple[int, int, int]]:
 
 def main() -> int:
     ap = argparse.ArgumentParser(description=__doc__.split("\n")[0])
-    ap.add_argument("--out", default=str(ROOT / "gpurun_out" / "plan_sweep_mi355x.json"))
+    ap.add_argument("--out", default="sweep.json")
     args = ap.parse_args()
     sys.path.insert(0, str(PKG))
     import torch

@@ -366,7 +366,9 @@ def test_cpu_tensors_have_no_kernel(adapter):
 # Measured on MI355X (tests/plan_sweep.py): for 87 chunk geometries (TriangleMix and dense-companion chunks
 # of 64-12288 rows at prompts of 1024-131072 tokens) every forced (KV parts, tiles per item) plan was timed.
 # The planner's costs were fitted to the 52 geometries not marked held_out, checked on the other 35, then
-# fitted on all 87 (tests/plan_fit.py).
+# fitted on all 87 (tests/plan_fit.py).  The sweep was taken when the eight-wave kernel ran every plan; plans with
+# long items have since moved to the kernel with 64 rows per wave, which is faster on them.  So these tests hold the
+# planner to the measurements its costs come from, in the eight-wave kernel, and not to what a planned chunk takes now.
 SWEEP = json.loads((Path(__file__).parent / "plan_sweep_mi355x.json").read_text())
 sys.path.insert(0, str(Path(__file__).parent))
 import plan_sweep  # noqa: E402
@@ -388,15 +390,15 @@ def _loss(g):
                          ids=[f"{g['query_start']}+{g['query_tokens']}/{g['seq_len']}/{g['prompt_len']}"
                               for g in SWEEP["geometries"]])
 def test_planned_plan_is_near_the_fastest_measured(lib, g):
-    """The planner's choice is the fastest measured plan or close to it: at worst 9.3 % slower (the last
-    1024 rows of a 16384-token prompt), and within 1 % on 70 of the 87 chunks."""
+    """The planner's choice is the fastest measured plan or close to it, in the eight-wave kernel: at worst 9.3 %
+    slower (the last 1024 rows of a 16384-token prompt), and within 1 % on 70 of the 87 chunks."""
     planned, fastest = _loss(g)
     assert planned <= 1.10 * fastest
 
 
 def test_planner_loss_over_the_sweep(lib):
     """Summed over the 87 geometries the planned plans lose 43.5 us of the 6,533 us the chunks take at their
-    fastest (0.67 %): 12.8 us over the 52 first fitted on, 30.8 us over the 35 held out of that fit."""
+    fastest in the eight-wave kernel (0.67 %): 12.8 us over the 52 first fitted on, 30.8 us over the 35 held out of that fit."""
     fit = [_loss(g) for g in SWEEP["geometries"] if not g["held_out"]]
     held = [_loss(g) for g in SWEEP["geometries"] if g["held_out"]]
     assert len(fit) == 52 and len(held) == 35
